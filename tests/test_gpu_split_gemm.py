@@ -1,0 +1,83 @@
+"""fp32 products on the three-way bf16 split (gemm_split_kernel) against
+float64: the slab counts its pipeline treats apart (one to four slabs of 16 k,
+the k tail, the sign changes every 16 slabs), partial tiles of each
+configuration, values that overflow or are not finite, and the mean of its
+error over a long contraction."""
+
+import pytest
+import torch
+
+from torchsplinekan_amd import _C, _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(M, N, K, ta, tb, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    A = torch.randn(*((K, M) if ta else (M, K)), generator=g)
+    B = torch.randn(*((N, K) if tb else (K, N)), generator=g)
+    return (A.t() if ta else A), (B.t() if tb else B)
+
+
+def _check(A, B):
+    got = _C.matmul(A.cuda(), B.cuda()).cpu().double()
+    want = A.double() @ B.double()
+    # one rounding per slab, at most 16 in a slab's chain (six MFMAs, each two
+    # truncating steps, and the dropped products), of 2^-24 of the sum of
+    # magnitudes; 64 more for the split slices
+    bound = (A.shape[1] / 16 + 16 + 64) * 2.0 ** -24 * (A.double().abs() @ B.double().abs())
+    assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("K", [17, 32, 33, 47, 64, 79, 257, 272, 530])
+def test_slab_counts_and_tails(tile, ta, tb, K):
+    M, N = 129, 64 if tile == "256x64" else 131
+    with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+        _check(*_operands(M, N, K, ta, tb, seed=K))
+
+
+@pytest.mark.parametrize("shape", [(17, 17, 40), (255, 257, 48), (257, 63, 100), (1000, 301, 77)])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_partial_tiles(shape, ta, tb):
+    _check(*_operands(*shape, ta, tb, seed=sum(shape)))
+
+
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_non_finite_and_overflowing_values(tile, ta, tb):
+    """What fp32 arithmetic gives: infinities keep their sign, NaN stays NaN,
+    and a value whose parts overflow bf16 still has its product."""
+    M, N, K = 40, 40, 100
+    A, B = _operands(M, N, K, ta, tb)
+    B = B.abs() + 0.25
+    A, B = A.clone(), B.clone()
+    A[3, 5], A[7, 90] = float("inf"), -float("inf")
+    A[11, 2] = float("nan")
+    A[20] = 0.0
+    A[20, 7] = 3.4028234e38
+    B[7, 1] = 0.5
+    with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+        got = _C.matmul(A.cuda(), B.cuda()).cpu()
+    assert bool((got[3] == float("inf")).all()) and bool((got[7] == -float("inf")).all())
+    assert bool(got[11].isnan().all())
+    want = (A[20:21].double() @ B.double()).float()[0]    # one term a value: exact
+    assert torch.equal(got[20], want)
+    rest = [i for i in range(M) if i not in (3, 7, 11, 20)]
+    err = (got[rest].double() - A[rest].double() @ B.double()).abs()
+    assert bool((err <= (K + 8) * 2.0 ** -24 * (A[rest].double().abs() @ B.double().abs())).all())
+
+
+def test_error_has_no_mean():
+    """The MFMA's rounding towards minus infinity must not add up: over 65536
+    output values the mean error lies within five standard errors plus a
+    hundredth of the truncation's own mean (-3e-8 of a term's rms per slab,
+    K / 16 slabs, were it left in)."""
+    M = N = 256
+    K = 16384
+    A, B = _operands(M, N, K, False, True, seed=1)
+    with _lib.route("gemm_tile", 0):
+        err = _C.matmul(A.cuda(), B.cuda()).cpu().double() - A.double() @ B.double()
+    limit = 5 * float(err.std()) / (M * N) ** 0.5 + 0.01 * 3e-8 * (K / 16)
+    assert abs(float(err.mean())) < limit

@@ -8,28 +8,28 @@
 //   input    E[n,k]  = sum_o D[n,o] W[o,k]     (NN)
 // They replace the cuBLAS calls of csrc/kan_cuda.cu:521-529, 579-604.
 //
-// fp32 runs on gemm_pipe_kernel, a software-pipelined v_mfma_f32_32x32x2f32
-// main loop, in one of three tile configurations picked per problem by a
-// cost model (pick_cfg_f32):
+// fp32 runs on gemm_split_kernel: every operand value as the exact sum of
+// three bf16 values, six v_mfma_f32_32x32x16_bf16 per product, fp32 sums (see
+// there), in one of three tile configurations picked per problem by a cost
+// model (pick_cfg_f32):
 //   big    256x256 block tile, 8 waves of 128x64 (two waves per SIMD), one
 //          block per CU;
 //   small  128x128 block tile, 4 waves of 64x64, two blocks per CU (for
 //          problems with too few big tiles to fill the chip);
 //   narrow 256x64 block tile, 4 waves of 64x64, for outputs of at most 64
 //          columns.
-// A 256x256 tile over 4 waves of 128x128 (one wave per SIMD) can be forced
-// for comparison.
-// fp64 runs on gemm_kernel: 128x128 tile, 2x2 waves, v_mfma_f64_16x16x4f64.
+// fp64 runs on gemm_pipe_kernel (v_mfma_f64_16x16x4f64, 128x128 or 64x64
+// tiles) and, when its tiles are forced, on gemm_kernel.
 //
-// Operand slabs (BK deep) are staged through LDS with double buffering.  Each
-// operand keeps its global layout in LDS:
+// The fp64 kernels stage operand slabs (BK deep) through LDS with double
+// buffering.  Each operand keeps its global layout in LDS:
 //   K-contiguous operand  -> LDS [rows][BK+4]; a lane reads 4 consecutive k
-//                            with one 16-byte ds_read.  Within each k-group
-//                            of the MFMA the k order is permuted identically
-//                            for A and B (step s, lane group q uses
-//                            k = KG*g + 4q + s), which leaves the sum unchanged;
+//                            with one read.  Within each k-group of the MFMA
+//                            the k order is permuted identically for A and B
+//                            (step s, lane group q uses k = KG*g + 4q + s),
+//                            which leaves the sum unchanged;
 //   MN-contiguous operand -> LDS [BK][rows+4]; a lane reads one element.
-// Pipeline of gemm_pipe_kernel, per K slab kt (NG k-groups of 8):
+// Pipeline of gemm_pipe_kernel, per K slab kt (NG k-groups):
 //   group 0 issues the LDS stores of slab kt+1 (held in registers) and the
 //   global loads of slab kt+2, interleaved one-for-one with its MFMAs by
 //   scheduling-group barriers; every group reads the fragments of the next
@@ -60,6 +60,7 @@ constexpr int kPadMN = 4;
 constexpr int kGroupM = 8;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -114,15 +115,15 @@ struct Cfg {
   static_assert(BK % Mfma<T, MF>::kKG == 0, "slab must be whole k-groups");
 };
 
-// 256 x 256 block tiles: 8 waves of 128 x 64 (two per SIMD: while one wave
-// of a SIMD waits at the slab barrier or on its fragment reads, the other
-// issues MFMAs), or 4 waves of 128 x 128 (one per SIMD; only when forced).
-using CfgF32Big = Cfg<float, 256, 256, 32, 2, 4, 32, 1>;
-using CfgF32Big4 = Cfg<float, 256, 256, 32, 2, 2, 32, 1>;
-using CfgF32Small = Cfg<float, 128, 128, 32, 2, 2, 32, 2>;
+// fp32 (gemm_split_kernel): 256 x 256 block tiles, 8 waves of 128 x 64 (two
+// per SIMD: while one wave of a SIMD waits at the slab barrier, on its
+// fragment reads or on its VALU work, the other issues MFMAs)
+using CfgF32Big = Cfg<float, 256, 256, 16, 2, 4, 32, 1>;
+// 128 x 128, 4 waves of 64 x 64, two blocks per CU
+using CfgF32Small = Cfg<float, 128, 128, 16, 2, 2, 32, 2>;
 // Narrow outputs (N <= 64, e.g. a 64-wide layer): 4 waves stacked along M,
 // 64 x 64 each, so no wave computes padding columns.
-using CfgF32Narrow = Cfg<float, 256, 64, 32, 4, 1, 32, 1>;
+using CfgF32Narrow = Cfg<float, 256, 64, 16, 4, 1, 32, 2>;
 using CfgF64 = Cfg<double, 128, 128, 16, 2, 2, 16, 1>;
 // fp64, 256 x 128 block tiles: 8 waves of 64 x 64, two per SIMD (while one
 // wave waits at the slab barrier the other issues MFMAs)
@@ -135,10 +136,10 @@ using CfgF64Pipe = Cfg<double, 128, 128, 32, 2, 4, 16, 1>;
 // (a 64-wide layer's products fill half of a 128 x 128 tile)
 using CfgF64Small = Cfg<double, 64, 64, 32, 2, 2, 16, 2>;
 
-// Configurations that run on gemm_pipe_kernel (the rest on gemm_kernel).
+// fp64 configurations that run on gemm_pipe_kernel (the rest on gemm_kernel).
 template <class C>
 struct RunsPipe {
-  static constexpr bool value = std::is_same<typename C::T, float>::value || C::BK == 32;
+  static constexpr bool value = C::BK == 32;
 };
 
 template <typename T>
@@ -151,7 +152,7 @@ struct GemmParams {
   int64_t k_per_split;
   int64_t split_stride;
   int tiles_m, tiles_n, splits;
-  int vec;  // operands 16-byte aligned with leading dimensions % 4 == 0
+  int vec;  // operands 16-byte aligned with leading dimensions % 4 == 0 (fp64 kernels)
   int buf;  // a whole slab's byte offsets fit 31 bits (buffer-resource loads)
 };
 
@@ -174,13 +175,15 @@ __device__ __forceinline__ TileCoords tile_coords(const GemmParams<T>& p) {
   const int pid = xcd_remap(blockIdx.x, total);
   const int per_split = p.tiles_m * p.tiles_n;
   TileCoords tc;
-  tc.split = pid / per_split;
+  // (uniform values: the integer divisions run in vector registers, and a
+  // base address the compiler holds there would make every buffer load a loop)
+  tc.split = __builtin_amdgcn_readfirstlane(pid / per_split);
   const int t = pid - tc.split * per_split;
   const int group = kGroupM * p.tiles_n;
   const int first_m = (t / group) * kGroupM;
   const int gm = min(p.tiles_m - first_m, kGroupM);
-  const int tm = first_m + (t % group) % gm;
-  const int tn = (t % group) / gm;
+  const int tm = __builtin_amdgcn_readfirstlane(first_m + (t % group) % gm);
+  const int tn = __builtin_amdgcn_readfirstlane((t % group) / gm);
   tc.m0 = (int64_t)tm * C::BM;
   tc.n0 = (int64_t)tn * C::BN;
   tc.kbeg = (int64_t)tc.split * p.k_per_split;
@@ -217,35 +220,6 @@ struct SlabLoader {
       int64_t r, kk;
       coords(threadIdx.x + p * NT, row0, k0, r, kk);
       reg[p] = *reinterpret_cast<const Vec4<T>*>(KCONT ? src + r * ld + kk : src + kk * ld + r);
-    }
-  }
-
-  // Whole slab through a buffer resource (fp32).  A lane's byte offset
-  // within a slab is the same for every slab, and its chunks p lie a
-  // wave-uniform stride apart, so a load takes no per-lane address
-  // arithmetic: base (scalar, per slab) + voff (lane, set once) + p * stride
-  // (scalar soffset).  Needs NT to be a multiple of the chunks per row.
-  uint32_t voff;
-  static constexpr int64_t kStep = KCONT ? NT / (BK / 4) : NT / (ROWS / 4);  // rows (k) per p
-  __device__ __forceinline__ void init_buf(int64_t ld) {
-    static_assert(KCONT ? NT % (BK / 4) == 0 : NT % (ROWS / 4) == 0, "uniform chunk stride");
-    int64_t r, kk;
-    coords(threadIdx.x, 0, 0, r, kk);
-    voff = (uint32_t)((KCONT ? r * ld + kk : kk * ld + r) * (int64_t)sizeof(T));
-  }
-  __device__ __forceinline__ void load_buf(const T* __restrict__ src, int64_t ld, int64_t row0,
-                                           int64_t k0) {
-    static_assert(sizeof(T) == 4, "128-bit buffer loads of 4 fp32 values");
-    const T* base = KCONT ? src + row0 * ld + k0 : src + k0 * ld + row0;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(base), (short)0, -1, 0x00020000 /* gfx9 raw buffer, 32-bit data */);
-#pragma unroll
-    for (int p = 0; p < kPer; ++p) {
-      typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(
-          rs, (int)voff, (int)((int64_t)p * kStep * ld * (int64_t)sizeof(T)), 0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) reg[p].v[j] = __uint_as_float(v[j]);
     }
   }
 
@@ -434,7 +408,7 @@ __global__ __launch_bounds__(C::kThreads, C::MINB) void gemm_kernel(GemmParams<t
   store_tile<C, typename M::acc_t, AIL, BIL>(p, tc, acc, wm, wn, lane);
 }
 
-// ---- fp32: software-pipelined main loop ------------------------------------
+// ---- software-pipelined main loop (fp64); fp32 epilogues ------------------------------------
 
 template <int N_>
 struct IC {
@@ -771,14 +745,460 @@ __device__ __forceinline__ void ecomp_epilogue(const GemmParams<float>& p, const
   }
 }
 
+// Floats of one wave's side buffer in the epilogues (knot rows and samples).
+template <class C>
+struct EpiSide {
+  static constexpr int kFloats = 2 * C::BN * 36 / (C::WM * C::WN);
+};
+
+// ---- fp32 on bf16 MFMA: three-way split operands ---------------------------
+//
+// An fp32 value is the sum of three bf16 values, x = hi + mid + lo, exactly
+// (8 significant bits each, every part rounded to nearest, so mid <= 2^-9 |x|
+// and lo <= 2^-18 |x|).  A product of two such sums needs six bf16 products
+// to fp32 accuracy (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three
+// dropped ones are below 2^-26 of the product.  Every product of two bf16
+// values is exact in fp32 and the MFMA accumulates in fp32, so the result
+// carries the accumulation's rounding only.
+//
+// Accumulation: a 16-k slab's six MFMAs of a tile run as one chain from zero
+// (smallest parts first) and their result is added to the tile's sum, so the
+// long sum takes one rounding per 16 k.  With the six accumulated straight
+// into the sum it took about twelve, which at K = 14336 with a third of the
+// values non-zero (a basis operand) was more than the fp32 MFMA's one per
+// non-zero k: relative error against float64 1.73e-6, fp32 MFMA 1.32e-6, as
+// built 0.58e-6 (K = 1024, dense: 0.48, 0.58 and 0.16e-6).  The adds cost 5 %.
+//
+// Sign: the bf16 MFMA rounds its aligned terms towards minus infinity, so its
+// error has a mean, -3e-8 of a term per slab, that grows with the number of
+// slabs where the rounding of a sum grows with its square root (a parameter
+// product over 8192 samples came out 3.7e-6 off in the mean-heavy gradients
+// of a 4096 -> 256 layer, the fp32 MFMA 0.6e-6).  Every second run of
+// kSplitRun slabs therefore holds -A and the sums change sign with it, which
+// cancels the mean (odd K slices start with -A: a slice may be one run).  At
+// K = 8192 it falls from 1.6e-7 of the result's rms to below 1e-8.
+// (Subtracting every second slab's partial sum, an FMA by +-1, cost 5 %;
+// turning the sums costs one VALU operation a value every 16 slabs, 1.5 %.)
+//
+// What bounds it: the chip's power.  At 65536 x 1024 x 14336 the kernel runs
+// at 1.9 GHz (the fp32 MFMA kernel before it at 2.37) with the MFMA pipes 0.70
+// busy: 1.35 PFLOP/s of bf16, about what torch.mm reaches in bf16 on the same
+// card (1.17-1.41).  Measured against the fp32 MFMA kernel on one box:
+// forward 65536 x 1024 x 14336 12.63 -> 8.59 ms, input-side 65536 x 14336 x
+// 1024 13.09 -> 9.47, parameter 1024 x 14336 x 65536 12.71 -> 8.77 (152 ->
+// 224, 147 -> 203, 151 -> 219 TFLOP/s of fp32 work); odd sizes, 1000^3 with
+// K % 16 != 0: 0.143 -> 0.055 ms.
+//
+// Layout: operands are split on their way from registers to LDS (5.5 VALU
+// operations a value, hidden behind the MFMAs), so global memory holds fp32
+// only and either global layout becomes the K-contiguous rows the MFMA reads
+// with 16-byte loads.  Slabs are one MFMA deep (16 k; 48 KB for 256 + 256
+// rows) and double buffered.  Per slab a wave keeps B's fragments and two
+// rows of A's; a slab's stores, the loads of the slab after next and the
+// adds are spread over its tiles, and the barrier that publishes the next
+// slab sits before the last tile, whose MFMAs cover the next first reads.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// (lambdas used at several places are not always inlined otherwise, and the
+// accumulators then live in memory)
+#define KAN_INLINE_LAMBDA __attribute__((always_inline))
+
+constexpr int kSplitBK = 16;        // k depth of a slab: one 32x32x16 MFMA
+constexpr int kSplitRowBytes = 32;  // 16 bf16 values of one plane
+constexpr int kSplitRun = 16;       // slabs between sign changes (a power of two)
+
+__device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(unsigned int u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned int u) {
+  return __uint_as_float(u & 0xffff0000u);
+}
+
+// Byte offset of the 16-byte chunk (row, 8-k half) in a plane: rows of 32
+// bytes, the two halves exchanged in every second group of 8 rows, so that
+// 16 consecutive rows of one half fall in distinct banks.
+__device__ __forceinline__ int split_chunk(int row, int half) {
+  return row * kSplitRowBytes + ((half ^ ((row >> 3) & 1)) << 4);
+}
+
+// Global -> register -> LDS staging of one operand slab (ROWS x 16).  A task
+// is one row's 8 consecutive k: two 16-byte loads of a K-contiguous operand,
+// eight 4-byte loads (consecutive lanes on consecutive rows) of an
+// MN-contiguous one; either way its three parts go to LDS as one 16-byte
+// store each.  Where the slab has fewer tasks than the block has threads,
+// the threads past the last task repeat an earlier one (same values to the
+// same place).
+template <int ROWS, bool KCONT, int NT>
+struct SplitLoader {
+  static constexpr int kTasks = 2 * ROWS;
+  static constexpr int kPer = kTasks >= NT ? kTasks / NT : 1;
+  static_assert(kTasks >= NT ? kTasks % NT == 0 : NT % kTasks == 0, "tasks split evenly");
+  static_assert(NT % ROWS == 0 && NT % 2 == 0, "uniform task strides");
+  static constexpr int kPlane = ROWS * kSplitRowBytes;
+  float reg[kPer][8];
+  int row, half;  // of task 0; task p is p * (NT / 2) rows or p * (NT / ROWS) halves on
+  uint32_t voff[KCONT ? kPer : 1];  // byte offset in a slab
+
+  // Rows past the operand's last (nrow - 1 of this tile) repeat that row:
+  // their products are never stored.
+  __device__ __forceinline__ void init(int64_t ld, int64_t nrow) {
+    const int t = kTasks >= NT ? (int)threadIdx.x : (int)threadIdx.x % kTasks;
+    row = KCONT ? t >> 1 : t % ROWS;
+    half = KCONT ? t & 1 : t / ROWS;
+#pragma unroll
+    for (int p = 0; p < (KCONT ? kPer : 1); ++p) {
+      const int64_t r = min((int64_t)row_of(p), nrow - 1);
+      voff[p] = (uint32_t)((KCONT ? r * ld + 8 * half : (int64_t)(8 * half) * ld + r) * 4);
+    }
+  }
+  __device__ __forceinline__ int row_of(int p) const { return KCONT ? row + p * (NT / 2) : row; }
+  __device__ __forceinline__ int half_of(int p) const {
+    return KCONT ? half : half + p * (NT / ROWS);
+  }
+
+  // A slab through a buffer resource: base (scalar, per slab) + voff (lane,
+  // set once) + a scalar offset per load.  TAIL: k from kend on reads as zero
+  // (an offset outside the resource).
+  template <bool TAIL>
+  __device__ __forceinline__ void load_buf(const float* __restrict__ src, int64_t ld, int64_t row0,
+                                           int64_t k0, int64_t kend) {
+    const float* base = KCONT ? src + row0 * ld + k0 : src + k0 * ld + row0;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(base), (short)0, 0x7fffffff, 0x00020000 /* raw buffer, 32-bit data */);
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      if constexpr (KCONT && !TAIL) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff[p] + 16 * h, 0, 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) reg[p][4 * h + j] = __uint_as_float(v[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          uint32_t off = KCONT ? voff[p] + 4 * j : voff[0];
+          if (TAIL && k0 + 8 * half_of(p) + j >= kend) off = 0x80000000u;
+          reg[p][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              rs, (int)off,
+              KCONT ? 0 : (int)(((int64_t)p * (NT / ROWS) * 8 + j) * ld * 4), 0));
+        }
+      }
+    }
+  }
+
+  // A slab whose offsets do not fit a buffer resource: 64-bit addresses,
+  // clamped into the operand, zero outside it.
+  __device__ __forceinline__ void load_guarded(const float* __restrict__ src, int64_t ld,
+                                               int64_t row0, int64_t rows, int64_t k0,
+                                               int64_t kend) {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int64_t r = row0 + row_of(p), kb = k0 + 8 * half_of(p);
+      const int64_t rc = r < rows ? r : rows - 1;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int64_t kj = kb + j, kc = kj < kend ? kj : kend - 1;
+        const float v = KCONT ? src[rc * ld + kc] : src[kc * ld + rc];
+        reg[p][j] = (r < rows && kj < kend) ? v : 0.0f;
+      }
+    }
+  }
+
+  // The values times -1 where flip is the sign bit (0: as they are).
+  __device__ __forceinline__ void store(char* __restrict__ lds, uint32_t flip) const {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      u32x4 hi, mid, lo;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x0 = __uint_as_float(__float_as_uint(reg[p][2 * j]) ^ flip);
+        const float x1 = __uint_as_float(__float_as_uint(reg[p][2 * j + 1]) ^ flip);
+        const unsigned int h = pack_bf16(x0, x1);
+        const float r0 = x0 - bf16_lo(h), r1 = x1 - bf16_hi(h);
+        const unsigned int m = pack_bf16(r0, r1);
+        hi[j] = h;
+        mid[j] = m;
+        lo[j] = pack_bf16(r0 - bf16_lo(m), r1 - bf16_hi(m));
+      }
+      char* dst = lds + split_chunk(row_of(p), half_of(p));
+      *reinterpret_cast<u32x4*>(dst) = hi;
+      *reinterpret_cast<u32x4*>(dst + kPlane) = mid;
+      *reinterpret_cast<u32x4*>(dst + 2 * kPlane) = lo;
+    }
+  }
+};
+
+// The same tile in plain fp32 (v_mfma_f32_32x32x2f32, guarded loads, one
+// slab at a time): the result where a split product is not finite.  A part
+// of an infinite or nearly overflowing value times a part of the opposite
+// sign gives NaN or infinity where the fp32 product has a value, so a block
+// that meets a non-finite sum evaluates its tile again here, and what the
+// caller sees is the fp32 arithmetic's infinity, NaN or number.
+template <class C, bool AK, bool BKC>
+__device__ __forceinline__ void fp32_tile(const GemmParams<float>& p, const TileCoords& tc,
+                                          f32x16 (&acc)[C::FM][C::FN], float* lds, int wm, int wn,
+                                          int lane) {
+  typedef Mfma<float, 32> M;
+  constexpr int BM = C::BM, BN = C::BN, BK = C::BK, NT = C::kThreads;
+  float* la_lds = lds;
+  float* lb_lds = lds + Slab<BM, BK, AK>::kElems;
+  SlabLoader<float, BM, BK, AK, NT> la;
+  SlabLoader<float, BN, BK, BKC, NT> lb;
+  const int rl = M::row(lane), q = M::kq(lane);
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+#pragma unroll 1
+  for (int kt = 0; kt < tc.nkt; ++kt) {
+    const int64_t k0 = tc.kbeg + (int64_t)kt * BK;
+    __syncthreads();
+    la.load_guarded(p.A, p.lda, tc.m0, p.M, k0, tc.kend);
+    la.store(la_lds);
+    lb.load_guarded(p.B, p.ldb, tc.n0, p.N, k0, tc.kend);
+    lb.store(lb_lds);
+    __syncthreads();
+#pragma unroll 1
+    for (int g = 0; g < BK / M::kKG; ++g) {
+      float fa[C::FM][4], fb[C::FN][4];
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i)
+        read_frag<float, BM, BK, AK>(la_lds, wm * C::TM + i * 32 + rl, M::kofs(g, q), fa[i]);
+#pragma unroll
+      for (int j = 0; j < C::FN; ++j)
+        read_frag<float, BN, BK, BKC>(lb_lds, wn * C::TN + j * 32 + rl, M::kofs(g, q), fb[j]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+          for (int j = 0; j < C::FN; ++j) acc[i][j] = M::mma(fa[i][s], fb[j][s], acc[i][j]);
+    }
+  }
+}
+
 template <class C, bool AK, bool BKC, int EPIK>
+struct SplitLds {
+  static constexpr int kBuf = (C::BM + C::BN) * 3 * kSplitRowBytes;
+  static constexpr int kSlabs = 2 * kBuf;
+  static constexpr int kTile =
+      4 * (Slab<C::BM, C::BK, AK>::kElems + Slab<C::BN, C::BK, BKC>::kElems);
+  static constexpr int kStage = 4 * C::WM * C::WN * 32 * (C::TN + 1);
+  static constexpr int kSide = EpiSide<C>::kFloats * 4 * C::WM * C::WN;
+  static constexpr int kBase = kSlabs > kTile ? kSlabs : kTile;
+  static constexpr int kBytes = EPIK == 0 || kStage + kSide < kBase ? kBase : kStage + kSide;
+};
+
+template <class C, bool AK, bool BKC, int EPIK>
+__global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+gemm_split_kernel(GemmParams<float> p, DxParams e) {
+  constexpr int BM = C::BM, BN = C::BN, NT = C::kThreads;
+  constexpr int FM = C::FM, FN = C::FN;
+  typedef SplitLoader<BM, AK, NT> LA;
+  typedef SplitLoader<BN, BKC, NT> LB;
+  typedef SplitLds<C, AK, BKC, EPIK> Lds;
+  static_assert(C::BK == kSplitBK, "one MFMA deep");
+  __shared__ __align__(16) char lds[Lds::kBytes];
+
+  const TileCoords tc = tile_coords<C>(p);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wm = wave / C::WN, wn = wave % C::WN;
+
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+  LA la;
+  LB lb;
+  la.init(p.lda, p.M - tc.m0);
+  lb.init(p.ldb, p.N - tc.n0);
+  const int fofs = split_chunk(lane & 31, lane >> 5);
+  const int aofs = fofs + wm * C::TM * kSplitRowBytes;
+  const int bofs = fofs + 3 * LA::kPlane + wn * C::TN * kSplitRowBytes;
+  // fragments, parts hi, mid, lo: A by the parity of the tile row, B whole
+  bf16x8 af[2][3], bf[FN][3];
+  f32x16 tmp[2];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) tmp[1][v] = 0.0f;
+  auto read_a = [&](const char* buf, int i) KAN_INLINE_LAMBDA {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      af[i & 1][q] = *reinterpret_cast<const bf16x8*>(buf + aofs + q * LA::kPlane +
+                                                      i * 32 * kSplitRowBytes);
+  };
+  auto read_b = [&](const char* buf, int j) KAN_INLINE_LAMBDA {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      bf[j][q] = *reinterpret_cast<const bf16x8*>(buf + bofs + q * LB::kPlane +
+                                                  j * 32 * kSplitRowBytes);
+  };
+  auto product = [&](const bf16x8 (&a)[3], const bf16x8 (&b)[3]) {
+    f32x16 t;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+    t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], t, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], t, 0, 0, 0);
+  };
+  // mode: 0 = guarded (64-bit addresses), 1 = buffer loads of a whole slab,
+  // 2 = buffer loads, the last slab's k tail read as zero
+  auto gload_a = [&](int slab, auto mode_c) KAN_INLINE_LAMBDA {
+    constexpr int kMode = decltype(mode_c)::value;
+    const int64_t k0 = tc.kbeg + (int64_t)slab * kSplitBK;
+    if constexpr (kMode == 0) la.load_guarded(p.A, p.lda, tc.m0, p.M, k0, tc.kend);
+    else la.template load_buf<kMode == 2>(p.A, p.lda, tc.m0, k0, tc.kend);
+  };
+  auto gload_b = [&](int slab, auto mode_c) KAN_INLINE_LAMBDA {
+    constexpr int kMode = decltype(mode_c)::value;
+    const int64_t k0 = tc.kbeg + (int64_t)slab * kSplitBK;
+    if constexpr (kMode == 0) lb.load_guarded(p.B, p.ldb, tc.n0, p.N, k0, tc.kend);
+    else lb.template load_buf<kMode == 2>(p.B, p.ldb, tc.n0, k0, tc.kend);
+  };
+  // The sign note above: after every kSplitRun slabs the sums and the partial
+  // sum not yet added change sign, and the slabs that follow hold -A (or A
+  // again); `turned` is whether the sums are negated.
+  auto turned = [&](int kt) KAN_INLINE_LAMBDA { return (kt / kSplitRun + tc.split) & 1; };
+  auto negate = [&]() KAN_INLINE_LAMBDA {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = -acc[i][j];
+    tmp[1] = -tmp[1];
+  };
+  auto turn = [&](int kt) KAN_INLINE_LAMBDA {
+    if ((kt + 1) % kSplitRun == 0) negate();
+  };
+  constexpr int kTiles = FM * FN;
+  static_assert(FM % 2 == 0 && FN % 2 == 0, "the fragment and partial-sum parities repeat per slab");
+  auto slab = [&](int kt, auto store_c, auto load_c, auto full_c) KAN_INLINE_LAMBDA {
+    constexpr bool STORE = decltype(store_c)::value != 0;  // (there is a slab kt + 1)
+    constexpr bool LOAD = decltype(load_c)::value != 0;
+    const char* cur = lds + (kt & 1) * Lds::kBuf;
+    char* nxt = lds + ((kt + 1) & 1) * Lds::kBuf;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      const int i = t / FN, j = t % FN, u = (t + kTiles - 1) % kTiles;
+      if (t == 0) {
+#pragma unroll
+        for (int jj = 1; jj < FN; ++jj) read_b(cur, jj);
+      }
+      if (j == 0 && i + 1 < FM) read_a(cur, i + 1);
+      if (STORE && t == kTiles - 1) {
+        __syncthreads();
+        read_a(nxt, 0);
+        read_b(nxt, 0);
+      }
+      if (STORE && t == 0) {
+        la.store(nxt, (uint32_t)turned(kt + 1) << 31);
+        if (LOAD) gload_a(kt + 2, full_c);
+      }
+      if (STORE && t == kTiles / 2) {
+        lb.store(nxt + 3 * LA::kPlane, 0);
+        if (LOAD) gload_b(kt + 2, full_c);
+      }
+      tmp[t & 1] = product(af[i & 1], bf[j]);
+      acc[u / FN][u % FN] += tmp[(t + 1) & 1];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // body: the load mode of every slab but the last, tail: the last one's
+  auto run = [&](auto body_c, auto tail_c) KAN_INLINE_LAMBDA {
+    if (tc.nkt > 1) {
+      gload_a(0, body_c);
+      gload_b(0, body_c);
+    } else {
+      gload_a(0, tail_c);
+      gload_b(0, tail_c);
+    }
+    la.store(lds, (uint32_t)turned(0) << 31);
+    lb.store(lds + 3 * LA::kPlane, 0);
+    if (tc.nkt > 2) {
+      gload_a(1, body_c);
+      gload_b(1, body_c);
+    } else if (tc.nkt > 1) {
+      gload_a(1, tail_c);
+      gload_b(1, tail_c);
+    }
+    __syncthreads();
+    read_a(lds, 0);
+    read_b(lds, 0);
+    int kt = 0;
+    while (kt + 3 < tc.nkt) {  // (run by run: a test per slab would be if-converted)
+      const int end = min(tc.nkt - 3, kt + kSplitRun);
+      for (; kt < end; ++kt) slab(kt, IC<1>(), IC<1>(), body_c);
+      if (kt % kSplitRun == 0) negate();
+    }
+    if (kt + 2 < tc.nkt) {
+      slab(kt, IC<1>(), IC<1>(), tail_c);
+      turn(kt);
+      ++kt;
+    }
+    if (kt + 1 < tc.nkt) {
+      slab(kt, IC<1>(), IC<0>(), tail_c);
+      turn(kt);
+      ++kt;
+    }
+    slab(kt, IC<0>(), IC<0>(), tail_c);
+    acc[FM - 1][FN - 1] += tmp[1];
+    if (turned(kt)) negate();
+  };
+  if (tc.nkt > 0) {
+    if (p.buf) run(IC<1>(), IC<2>());
+    else run(IC<0>(), IC<0>());
+  }
+  // v * 0 is 0 for a finite v and NaN otherwise
+  float probe = 0.0f;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) probe = __builtin_fmaf(acc[i][j][v], 0.0f, probe);
+  __syncthreads();  // every wave is done with the slab buffers
+  int* flags = reinterpret_cast<int*>(lds);
+  const bool bad_wave = __any(probe != 0.0f);
+  if (lane == 0) flags[wave] = bad_wave ? 1 : 0;
+  __syncthreads();
+  int bad = 0;
+#pragma unroll
+  for (int w = 0; w < C::WM * C::WN; ++w) bad |= flags[w];
+  if (__builtin_amdgcn_readfirstlane(bad) != 0)
+    fp32_tile<C, AK, BKC>(p, tc, acc, reinterpret_cast<float*>(lds), wm, wn, lane);
+  if constexpr (EPIK == 0) {
+    (void)e;
+    store_tile<C, f32x16>(p, tc, acc, wm, wn, lane);
+  } else {
+    float* stage = reinterpret_cast<float*>(lds);
+    float* side = reinterpret_cast<float*>(lds + Lds::kStage);
+    constexpr int kSide = EpiSide<C>::kFloats;
+    static_assert(kSide + 512 <= 8192, "div_small covers the side buffer's indices");
+    __syncthreads();  // every wave has read the flags
+    if constexpr (EPIK > 0)
+      dx_epilogue<C, EPIK>(p, e, tc, acc, stage, side, kSide, wave, wm, wn, lane);
+    else
+      ecomp_epilogue<C, -EPIK>(p, e, tc, acc, stage, side, kSide, wave, wm, wn, lane);
+  }
+}
+
+template <class C, bool AK, bool BKC>
 __global__ __launch_bounds__(C::kThreads, C::MINB) void gemm_pipe_kernel(
-    GemmParams<typename C::T> p, DxParams e) {
+    GemmParams<typename C::T> p) {
   typedef typename C::T T;
   typedef Mfma<T, C::MF> M;
-  // fp32 loads whole slabs through buffer resources; fp64 (a four-element
-  // chunk is 32 bytes) through plain 16-byte loads
-  constexpr bool kF32 = std::is_same<T, float>::value;
   constexpr int BM = C::BM, BN = C::BN, BK = C::BK, NT = C::kThreads;
   constexpr int FM = C::FM, FN = C::FN, NG = BK / M::kKG;
   static_assert(NG % 2 == 0, "slab must hold an even number of k-groups");
@@ -841,14 +1261,10 @@ __global__ __launch_bounds__(C::kThreads, C::MINB) void gemm_pipe_kernel(
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = M::mma(fa[slot][i][s], fb[slot][j][s], acc[i][j]);
   };
-  // full_c: 1 = whole slabs through buffer resources, 0 = edge slabs
-  // (guarded; also whole slabs whose offsets do not fit a buffer resource)
+  // full_c: 1 = whole slabs, 0 = edge slabs (guarded)
   auto gload = [&](int slab, auto full_c) {
     const int64_t k0 = tc.kbeg + (int64_t)slab * BK;
-    if constexpr (decltype(full_c)::value == 1 && kF32) {
-      la.load_buf(p.A, p.lda, tc.m0, k0);
-      lb.load_buf(p.B, p.ldb, tc.n0, k0);
-    } else if constexpr (decltype(full_c)::value == 1) {
+    if constexpr (decltype(full_c)::value == 1) {
       la.load_full(p.A, p.lda, tc.m0, k0);
       lb.load_full(p.B, p.ldb, tc.n0, k0);
     } else {
@@ -891,10 +1307,6 @@ __global__ __launch_bounds__(C::kThreads, C::MINB) void gemm_pipe_kernel(
     }
   };
   auto run = [&](auto full_c) {
-    if constexpr (decltype(full_c)::value == 1 && kF32) {
-      la.init_buf(p.lda);
-      lb.init_buf(p.ldb);
-    }
     gload(0, full_c);
     la.store(lds_a[0]);
     lb.store(lds_b[0]);
@@ -910,28 +1322,12 @@ __global__ __launch_bounds__(C::kThreads, C::MINB) void gemm_pipe_kernel(
     slab(kt, IC<0>(), IC<0>(), IC<0>(), full_c, IC<-1>());
   };
   if (tc.nkt > 0) {
-    const bool full = p.vec && (p.buf || !kF32) && (tc.m0 + BM <= p.M) && (tc.n0 + BN <= p.N) &&
+    const bool full = p.vec && (tc.m0 + BM <= p.M) && (tc.n0 + BN <= p.N) &&
                       ((tc.kend - tc.kbeg) % BK == 0);
     if (full) run(IC<1>());
     else run(IC<0>());
   }
-  if constexpr (EPIK == 0) {
-    (void)e;
-    store_tile<C, typename M::acc_t, AIL, BIL>(p, tc, acc, wm, wn, lane);
-  } else {
-    static_assert(kF32, "the epilogues are fp32");
-    static_assert(!AIL && !BIL, "the epilogues read the accumulators in tile order");
-    static_assert(C::WM * C::WN * 32 * (C::TN + 1) <= 2 * SA::kElems,
-                  "dx staging must fit in the A slab buffers");
-    constexpr int kSide = 2 * SB::kElems / (C::WM * C::WN);
-    static_assert(kSide + 512 <= 8192, "div_small covers the side buffer's indices");
-    __syncthreads();  // every wave is done with the slab buffers
-    if constexpr (EPIK > 0)
-      dx_epilogue<C, EPIK>(p, e, tc, acc, &lds_a[0][0], &lds_b[0][0], kSide, wave, wm, wn, lane);
-    else
-      ecomp_epilogue<C, -EPIK>(p, e, tc, acc, &lds_a[0][0], &lds_b[0][0], kSide, wave, wm, wn,
-                               lane);
-  }
+  store_tile<C, typename M::acc_t, AIL, BIL>(p, tc, acc, wm, wn, lane);
 }
 
 // dx[n, i] = (part[n, i, 0] + part[n, i, 1]) (+ part[n, i, 2])
@@ -954,27 +1350,26 @@ bool vec_ok(const T* ptr, int64_t ld) {
 // ---- planning ----------------------------------------------------------------
 
 // Cost model of the fp32 tile configurations, fitted to a sweep of every
-// configuration and split count over the products of BASELINE's workloads
-// (c2's first layer, c3's and c5's parameter products, c4's and c5's
-// forward products) on MI355X.  The dispatcher spreads workgroups over CUs,
-// so the busiest CU runs ceil(tiles / CUs) blocks one after another (two
-// small blocks that share a CU run at half speed each, the same total);
-// a block costs its MFMA work at the configuration's sustained efficiency
-// plus a fixed start-up and write-out time.  The 128 x 128 tile loses most
-// of its efficiency when it runs alone on a CU (one wave per SIMD: the slab
-// barriers idle the MFMA pipes), which is why the earlier whole-wave model
-// (eff 0.85 at two blocks per CU, a 256-k overhead) split c2's and c5's
-// products onto small tiles that ran 10-30 % slower than the 256 x 256 tile
-// with more splits, and c3's parameter product 4 ways instead of 8.
+// configuration and split count (1..64) over 22 products on MI355X: the
+// three products of 784 -> 256, 256 -> 256, 1024 -> 1024, 512 -> 512, 512 ->
+// 64 and 4096 -> 256 layers, small batches and odd sizes (fit error 8 % rms
+// for the first two, 12 % for the narrow one; the choice it makes costs at
+// most 11 % over the best of the sweep, 2 % on average).  The dispatcher
+// spreads workgroups over CUs, so the busiest CU runs ceil(tiles / CUs)
+// blocks one after another (two small blocks that share a CU run at half
+// speed each, the same total); a block costs its MFMA work at the
+// configuration's sustained rate plus a fixed start-up and write-out time.
+// Rates are in units of the FP32 MFMA peak (the split products run above
+// it), lower on a full chip, where the clock drops under the bf16 load.
 struct CfgModel {
   int bm, bn, bk;
-  double eff;       // sustained fraction of the per-CU peak, blocks sharing CUs
+  double eff;       // sustained rate, blocks sharing CUs
   double eff_lone;  // the same when every block has a CU of its own
   double block_s;   // fixed seconds per block (start-up, epilogue)
 };
-constexpr CfgModel kModelF32[4] = {
-    {256, 256, 32, 0.89, 0.89, 5e-6}, {128, 128, 32, 0.88, 0.40, 10e-6},
-    {256, 64, 32, 0.75, 0.75, 5e-6}, {256, 256, 32, 0.89, 0.89, 5e-6}};
+constexpr CfgModel kModelF32[3] = {
+    {256, 256, kSplitBK, 1.50, 1.75, 10e-6}, {128, 128, kSplitBK, 1.35, 1.15, 5e-6},
+    {256, 64, kSplitBK, 0.85, 0.90, 2e-6}};
 constexpr double kPeakPerCuF32 = 157.3e12 / 256.0;  // FP32 MFMA flop/s per CU
 constexpr double kStreamBytesPerS = 5.0e12;          // split-K partial-sum traffic
 
@@ -1028,14 +1423,16 @@ double est_seconds_f64(const CfgModelF64& c, int64_t M, int64_t N, int64_t K, in
 }
 
 // Forced fp32 tile configuration (route KAN_ROUTE_GEMM_TILE: 0 big, 1 small,
-// 2 narrow, 3 the 4-wave 256x256), or -1 to leave the choice to the cost
-// model.
-int forced_cfg_f32() { return kan_hip_get_route(KAN_ROUTE_GEMM_TILE); }
+// 2 narrow; 3, a float64 tile, leaves fp32 on the big one), or -1 to leave
+// the choice to the cost model.
+int forced_cfg_f32() {
+  const int r = kan_hip_get_route(KAN_ROUTE_GEMM_TILE);
+  return r == 3 ? 0 : r;
+}
 
 // fp64 configuration (0 = 256 x 128 with 8 waves, 1 = 128 x 128 with 4,
 // 2 = the pipelined 128 x 128 x 32, 3 = the pipelined 64 x 64 x 32) for a
-// split count; the route forces 0 for "256", 1 for "128", 2 for "256x64"
-// and 3 for "256w4" (the fp32 tiles' values).
+// split count; the route's values 0 to 3 force them.
 int pick_cfg_f64(int64_t M, int64_t N, int64_t K, int splits, int64_t cus = 0) {
   const int forced = kan_hip_get_route(KAN_ROUTE_GEMM_TILE);
   if (forced >= 0 && forced <= 3) return forced;
@@ -1055,9 +1452,8 @@ int pick_cfg_f64(int64_t M, int64_t N, int64_t K, int splits, int64_t cus = 0) {
   return best;
 }
 
-// fp32 configuration (0 = big, 1 = small, 2 = narrow, 3 = 4-wave big, only
-// when forced) for a given split count; the narrow one only where N fits its
-// 64 columns.
+// fp32 configuration (0 = big, 1 = small, 2 = narrow) for a given split
+// count; the narrow one only where N fits its 64 columns.
 int pick_cfg_f32(int64_t M, int64_t N, int64_t K, int splits, int64_t cus = 0) {
   const int forced = forced_cfg_f32();
   if (forced >= 0) return forced;
@@ -1092,11 +1488,15 @@ int launch_cfg(GemmParams<typename C::T> p, int splits, hipStream_t st, const Dx
     return span * (int64_t)sizeof(typename C::T) < (int64_t)1 << 31;
   };
   p.buf = span_ok(AK, C::BM, p.lda) && span_ok(BKC, C::BN, p.ldb);
-  if constexpr (RunsPipe<C>::value) {
+  if constexpr (std::is_same<typename C::T, float>::value) {
     DxParams e{};
     if (dx != nullptr) e = *dx;
-    hipLaunchKernelGGL((gemm_pipe_kernel<C, AK, BKC, EPIK>), dim3((unsigned)blocks),
+    hipLaunchKernelGGL((gemm_split_kernel<C, AK, BKC, EPIK>), dim3((unsigned)blocks),
                        dim3(C::kThreads), 0, st, p, e);
+  } else if constexpr (RunsPipe<C>::value) {
+    (void)dx;
+    hipLaunchKernelGGL((gemm_pipe_kernel<C, AK, BKC>), dim3((unsigned)blocks),
+                       dim3(C::kThreads), 0, st, p);
   } else {
     (void)dx;
     hipLaunchKernelGGL((gemm_kernel<C, AK, BKC>), dim3((unsigned)blocks), dim3(C::kThreads), 0,
@@ -1120,8 +1520,7 @@ int launch_layout(int layout, const GemmParams<typename C::T>& p, int splits, hi
 // share of the B slab buffers; exact, by walking the blocks of the row.
 template <class C>
 bool dx_cfg_fits(int64_t N, int64_t I, int R, int nk, bool has_base) {
-  typedef Slab<C::BN, C::BK, true> SB;
-  constexpr int64_t kSide = 2 * SB::kElems / (C::WM * C::WN);
+  constexpr int64_t kSide = EpiSide<C>::kFloats;
   if (R > C::TN) return false;  // a feature's columns meet at most two blocks
   const int64_t ksp = I * R;
   for (int64_t c0 = 0; c0 < N; c0 += C::TN)
@@ -1140,8 +1539,7 @@ int launch_dx_cfg(const GemmParams<float>& p, const DxParams& e, int k, hipStrea
 // a window crossing blocks is completed by each of them).
 template <class C>
 bool ecomp_cfg_fits(int64_t N, int64_t I, int R, int nk, bool has_base) {
-  typedef Slab<C::BN, C::BK, true> SB;
-  constexpr int64_t kSide = 2 * SB::kElems / (C::WM * C::WN);
+  constexpr int64_t kSide = EpiSide<C>::kFloats;
   const int64_t ksp = I * R;
   for (int64_t c0 = 0; c0 < N; c0 += C::TN) {
     const DxBlock b(c0, N, ksp, R, C::TN, has_base);
@@ -1605,7 +2003,6 @@ int launch_gemm(int layout, int64_t M, int64_t N, int64_t K, const T* A, int64_t
   } else if constexpr (std::is_same<T, float>::value) {
     const int cfg = pick_cfg_f32(M, N, K, splits < 1 ? 1 : splits);
     if (cfg == 0) rc = launch_layout<CfgF32Big>(layout, p, splits, st);
-    else if (cfg == 3) rc = launch_layout<CfgF32Big4>(layout, p, splits, st);
     else if (cfg == 2) rc = launch_layout<CfgF32Narrow>(layout, p, splits, st);
     else rc = launch_layout<CfgF32Small>(layout, p, splits, st);
   } else {
@@ -1692,7 +2089,6 @@ bool gemm_dx_supported(int64_t M, int64_t N, int64_t K, int64_t I, int G, int k,
   const int R = G + k, nk = G + 2 * k + 1;
   const int cfg = pick_cfg_f32(M, N, K, 1);
   if (cfg == 0) return dx_cfg_fits<CfgF32Big>(N, I, R, nk, has_base);
-  if (cfg == 3) return dx_cfg_fits<CfgF32Big4>(N, I, R, nk, has_base);
   return dx_cfg_fits<CfgF32Small>(N, I, R, nk, has_base);
 }
 
@@ -1732,7 +2128,6 @@ int launch_gemm_dx(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
     TimedLaunch timed(kClassContraction, st, 2.0 * (double)M * (double)N * (double)K);
     const int cfg = pick_cfg_f32(M, N, K, 1);
     if (cfg == 0) rc = launch_dx_cfg<CfgF32Big>(p, e, k, st);
-    else if (cfg == 3) rc = launch_dx_cfg<CfgF32Big4>(p, e, k, st);
     else rc = launch_dx_cfg<CfgF32Small>(p, e, k, st);
     if (rc != KAN_OK) return rc;
     rc = check_launch("gemm_dx");
@@ -1753,7 +2148,6 @@ bool gemm_ecomp_supported(int64_t M, int64_t N, int64_t K, int64_t I, int G, int
   const int R = G + k, nk = G + 2 * k + 1;
   const int cfg = pick_cfg_f32(M, N, K, 1);
   if (cfg == 0) return ecomp_cfg_fits<CfgF32Big>(N, I, R, nk, has_base);
-  if (cfg == 3) return ecomp_cfg_fits<CfgF32Big4>(N, I, R, nk, has_base);
   return ecomp_cfg_fits<CfgF32Small>(N, I, R, nk, has_base);
 }
 
@@ -1792,7 +2186,6 @@ int launch_gemm_ecomp(int64_t M, int64_t N, int64_t K, const float* A, int64_t l
   const int cfg = pick_cfg_f32(M, N, K, 1);
   int rc;
   if (cfg == 0) rc = launch_ecomp_cfg<CfgF32Big>(p, e, k, st);
-  else if (cfg == 3) rc = launch_ecomp_cfg<CfgF32Big4>(p, e, k, st);
   else rc = launch_ecomp_cfg<CfgF32Small>(p, e, k, st);
   if (rc != KAN_OK) return rc;
   return check_launch("gemm_ecomp");

@@ -70,7 +70,9 @@ int64_t kan_hip_get_basis_impl(void);
  *   KAN_ROUTE_FUSED_DX   (KAN_HIP_FUSED_DX)   0 off (default), 1 dx contracted
  *                        in the input-side product's epilogue
  *   KAN_ROUTE_COMPACT_E  (KAN_HIP_COMPACT_E)  -1 automatic (R >= 25, default),
- *                        0 never, 1 always: span-window form of E
+ *                        0 never, 1 always: span-window form of E; -1 also
+ *                        lets rows of R >= 40 take the span-window products
+ *                        (as -1 of GEMM_TILE and 0 of FUSED_DX do)
  *   KAN_ROUTE_EDGE_FUSED (KAN_HIP_EDGE_FUSED) 1 (default) both gradient sides
  *                        of the edge statistic in one kernel, 0 separate
  *   KAN_ROUTE_GEMM_TILE  (KAN_HIP_GEMM_TILE)  -1 cost model (default), 0 256x256

@@ -1,0 +1,102 @@
+"""Span-window products (kan_span.hip) of layers with many basis functions:
+forward, inference and input gradient against float64, at the fp32 parity bar
+(normwise 1e-5), over orders, output widths that fill no block, sample and
+feature counts that fill no tile or slice, with and without the base branch;
+and what they make of inputs and weights that are not finite."""
+
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from torchsplinekan_amd import _C, _lib
+from torchsplinekan_amd.reference_backend import compute_basis
+
+pytestmark = pytest.mark.gpu
+
+# n, I, O, G, k, base: shapes whose inference or input gradient (or both) the
+# rule gives to the span kernels
+SHAPES = [(8498, 187, 51, 65, 2, True), (3000, 333, 61, 66, 2, True),
+          (3001, 250, 259, 65, 3, False), (13220, 73, 19, 65, 1, True),
+          (1281, 1068, 461, 65, 1, True), (4500, 500, 61, 65, 2, False),
+          (4729, 948, 61, 65, 3, True)]
+
+
+def _workspace(fn, *args):
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(fn(*args, ctypes.byref(nbytes)))
+    return nbytes.value
+
+
+def _routes(n, I, O, G, k, base):
+    """Which of (inference, input gradient) run on the span kernels: those
+    whose workspace differs from the dense route's."""
+    out = []
+    for fn, args in ((_lib.LIB.kan_hip_infer_workspace, (0, n, I, O, G, k, int(base))),
+                     (_lib.LIB.kan_hip_backward_workspace, (0, n, I, O, G, k, int(base), 1, 0))):
+        auto = _workspace(fn, *args)
+        with _lib.route("compact_e", 1):
+            out.append(auto != _workspace(fn, *args))
+    return out
+
+
+def _layer(n, I, O, G, k, base, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    knots = torch.arange(-k, G + k + 1) * (2.0 / G) - 1.0
+    grid = knots + (torch.rand(I, G + 2 * k + 1, generator=g) - 0.5) * (0.8 / G)
+    x = (torch.rand(n, I, generator=g) * 2 - 1) * 1.15
+    bw = torch.randn(O, I, generator=g) if base else torch.empty(0)
+    sw = torch.randn(O, I, G + k, generator=g) * 0.1
+    sc = torch.rand(O, I, generator=g) + 0.5
+    return [t.cuda() for t in (x, grid, bw, sw, sc)]
+
+
+def _norm(u, v):
+    u, v = u.detach().double(), v.detach()
+    return float((u - v).norm() / v.norm())
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_span_products_match_float64(shape):
+    n, I, O, G, k, base = shape
+    assert any(_routes(*shape))
+    x, grid, bw, sw, sc = _layer(*shape)
+    D = torch.randn(n, O, generator=torch.Generator().manual_seed(1)).cuda()
+    xg = x.clone().requires_grad_()
+    y = _C.kan_apply(xg, grid, bw, sw, sc, k, True)
+    dx, = torch.autograd.grad(y, xg, D)
+    waug = _C.pack_weight(bw if base else None, sw, sc, k, True)
+    yi = _C.kan_infer(x, grid, waug, k, base)
+
+    xd = x.double().requires_grad_()
+    W = (sw * sc.unsqueeze(-1)).double().flatten(1)
+    want = torch.cat([compute_basis(xd[i:i + 512], grid.double(), k).flatten(1) @ W.t()
+                      for i in range(0, n, 512)])
+    if base:
+        want = want + F.silu(xd) @ bw.double().t()
+    wdx, = torch.autograd.grad(want, xd, D.double())
+    assert _norm(y, want.detach()) < 1e-5
+    assert _norm(yi, want.detach()) < 1e-5
+    assert _norm(dx, wdx) < 1e-5
+    assert torch.equal(yi, _C.kan_infer(x, grid, waug, k, base))    # fixed order of sums
+
+
+def test_span_inputs_and_weights_that_are_not_finite():
+    """As in the dense product: NaN or infinite inputs reach their row through
+    silu alone; a weight that is not finite reaches its output's every sample."""
+    shape = (3000, 333, 61, 66, 2, True)
+    assert _routes(*shape)[0]
+    x, grid, bw, sw, sc = _layer(*shape)
+    bw = bw.abs() + 0.1
+    x[5, 7], x[6, 8], x[7, 9] = float("nan"), float("inf"), 50.0
+    sw[3, 100, 20] = float("nan")
+    waug = _C.pack_weight(bw, sw, sc, 2, True)
+    y = _C.kan_infer(x, grid, waug, 2, True)
+    with _lib.route("compact_e", 1):     # the dense product
+        want = _C.kan_infer(x, grid, waug, 2, True)
+    assert torch.equal(y.isnan(), want.isnan()) and bool(y[5].isnan().all())
+    assert bool(y[:, 3].isnan().all())
+    assert torch.equal(y == float("inf"), want == float("inf"))
+    ok = want.isfinite()
+    assert _norm(y[ok], want[ok].double()) < 1e-5

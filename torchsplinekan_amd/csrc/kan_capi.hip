@@ -226,9 +226,60 @@ int need_ptr(const void* p, const char* who, const char* name) {
     if (kan_rc_ != KAN_OK) return kan_rc_; \
   } while (0)
 
+// Whether an fp32 layer's product runs on the span-window kernels
+// (kan_span.hip): the local basis, no route forced, and less estimated time
+// than the dense product, which costs R + 1 columns a feature where they cost
+// k + 2.
+constexpr int64_t kSpanMinR = 40;
+bool span_may(int64_t n, int64_t I, int64_t O, int64_t R) {
+  return R >= kSpanMinR && n > 0 && I > 0 && O > 0 && g_basis_impl.load() == 1 &&
+         kan_hip_get_route(KAN_ROUTE_COMPACT_E) == -1 &&
+         kan_hip_get_route(KAN_ROUTE_FUSED_DX) == 0 &&
+         kan_hip_get_route(KAN_ROUTE_GEMM_TILE) == -1;
+}
+// Where the lines lie (64 random layers of 23 to 68 basis functions, both ways
+// measured; the two estimates together are off by up to 20 %):
+//  * rows below 40 stay dense (at 23 the input gradient lost up to 28 %: 16628 x
+//    3297 -> 22, 2.71 against 1.95 ms);
+//  * inference and input gradient below 0.8 of the dense estimate: won by 1.03
+//    to 2.6 and 1.02 to 1.4 times there (8192 x 4096 -> 256, R = 68: 3.78
+//    against 6.85 and 4.24 against 7.64 ms), lost up to 10 % at 0.95;
+//  * the forward that keeps the basis up to 256 outputs, below 0.95: won by 1.04
+//    to 1.4 times (8192 x 4096 -> 256: 3.65 against 5.10 ms); above 256 outputs
+//    it lost up to 14 % (332 x 1699 -> 1038: 0.87 against 0.75 ms).
+constexpr double kSpanMargin = 0.8;
+constexpr double kSpanForwardMargin = 0.95;
+constexpr int64_t kSpanForwardMaxO = 256;
+constexpr double kSpanStream = 5e12;  // bytes/s of the passes beside the products
+// Forward with the basis kept: the same basis pass and weight packing either way.
+bool span_forward_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
+                       SpanPlan* pl) {
+  if (O > kSpanForwardMaxO || !span_may(n, I, O, R)) return false;
+  *pl = span_plan(n, I, O, R, k, false);
+  return pl->seconds < kSpanForwardMargin * gemm_seconds_f32(n, O, kaug);
+}
+// Inference: the dense product also writes the basis and reads it back; the
+// span product transposes the packed weight.
+bool span_infer_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
+                     SpanPlan* pl) {
+  if (!span_may(n, I, O, R)) return false;
+  *pl = span_plan(n, I, O, R, k, false);
+  return pl->seconds + 8.0 * (double)(kaug * O) / kSpanStream + 4e-6 <
+         kSpanMargin * (gemm_seconds_f32(n, O, kaug) + 4.0 * (double)(n * kaug) / kSpanStream);
+}
+// Input gradient: against the dense product and the pass over its windows.
+bool span_dx_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
+                  SpanPlan* pl) {
+  if (!span_may(n, I, O, R)) return false;
+  *pl = span_plan(n, I, O, R, k, true);
+  return pl->seconds < kSpanMargin * (gemm_seconds_f32(n, kaug, O) +
+                                      4.0 * (double)(n * I * (k + 4)) / 3e12);
+}
+
 struct BackwardPlan {
   int64_t R, ld, kaug;
-  bool need_x, need_params, fused_dx, compact_dx;
+  bool need_x, need_params, fused_dx, compact_dx, span_dx;
+  SpanPlan span;
   int splits;
   size_t waug_elems, e_elems, part_elems;
   size_t ew_elems;  // compact route: window values [n, I, k+1], then the base columns
@@ -245,11 +296,20 @@ inline int64_t infer_slice_cap(int64_t scratch_elems, int64_t aug_elems) {
 }
 
 template <typename T>
-void infer_plan(int64_t n, int64_t I, int64_t O, int64_t R, bool has_base, int64_t* ld,
-                int64_t* kaug, int64_t* aug_elems, int64_t* part_elems,
+void infer_plan(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, bool has_base, int64_t* ld,
+                int64_t* kaug, int64_t* aug_elems, int64_t* part_elems, SpanPlan* span,
                 int64_t scratch_elems = -1) {
   *ld = aug_width(I, R, has_base);
   *kaug = I * R + (has_base ? I : 0);
+  *span = SpanPlan{};
+  // (the allocation-free call's scratch is sized for the basis)
+  if (std::is_same<T, float>::value && scratch_elems < 0 &&
+      span_infer_wins(n, I, O, R, k, *kaug, span)) {
+    *aug_elems = round_up(*kaug * O, 64);  // the transposed weight
+    *part_elems = span->part_elems;
+    return;
+  }
+  span->v = 0;  // dense
   *aug_elems = round_up(n * *ld, 64);
   *part_elems = matmul_ws_elems<T>(kLayoutNT, n, O, *kaug,
                                    infer_slice_cap(scratch_elems, *aug_elems));
@@ -272,10 +332,12 @@ BackwardPlan plan_backward(int64_t n, int64_t I, int64_t O, int64_t G, int64_t k
   const bool local_f32 = std::is_same<T, float>::value && g_basis_impl.load() == 1;
   p.fused_dx = need_x && local_f32 && fused_dx_enabled() &&
                gemm_dx_supported(n, p.kaug, O, I, (int)G, (int)k, has_base);
-  p.compact_dx = need_x && local_f32 && !p.fused_dx && compact_e_wanted(p.R) &&
+  p.span_dx = need_x && local_f32 && span_dx_wins(n, I, O, p.R, k, p.kaug, &p.span);
+  p.compact_dx = need_x && local_f32 && !p.fused_dx && !p.span_dx && compact_e_wanted(p.R) &&
                  gemm_ecomp_supported(n, p.kaug, O, I, (int)G, (int)k, has_base);
   p.ew_elems = p.compact_dx ? (size_t)round_up(n * I * (k + 1), 64) : 0;
   p.e_elems = !need_x         ? 0
+              : p.span_dx    ? (size_t)round_up(p.span.part_elems, 64)
               : p.fused_dx   ? (size_t)(n * I * (has_base ? 3 : 2))
               : p.compact_dx ? p.ew_elems + (size_t)(has_base ? round_up(n * I, 64) : 0)
                              : (size_t)(n * p.ld);
@@ -288,11 +350,18 @@ BackwardPlan plan_backward(int64_t n, int64_t I, int64_t O, int64_t G, int64_t k
 // (few samples or outputs, long K: c5's layer, small networks) are split over
 // K and summed in a fixed order; large ones (c3) are not split.
 template <typename T>
-void forward_plan(int64_t n, int64_t I, int64_t O, int64_t R, bool has_base, int64_t* ld,
-                  int64_t* kaug, int64_t* waug_elems, int64_t* part_elems) {
+void forward_plan(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, bool has_base,
+                  int64_t* ld, int64_t* kaug, int64_t* waug_elems, int64_t* part_elems,
+                  SpanPlan* span) {
   *ld = aug_width(I, R, has_base);
   *kaug = I * R + (has_base ? I : 0);
-  *waug_elems = round_up(O * *ld, 64);
+  *waug_elems = round_up(O * *ld, 64);  // (the transposed weight [kaug, O] fits too)
+  *span = SpanPlan{};
+  if (std::is_same<T, float>::value && span_forward_wins(n, I, O, R, k, *kaug, span)) {
+    *part_elems = span->part_elems;
+    return;
+  }
+  span->v = 0;  // dense
   *part_elems = matmul_ws_elems<T>(kLayoutNT, n, O, *kaug);
 }
 
@@ -303,7 +372,8 @@ int forward_impl(const void* x, const void* grid, const void* bw, const void* sw
   const int64_t R = G + k;
   const bool has_base = bw != nullptr;
   int64_t ld, kaug, waug_elems, part_elems;
-  forward_plan<T>(n, I, O, R, has_base, &ld, &kaug, &waug_elems, &part_elems);
+  SpanPlan span;
+  forward_plan<T>(n, I, O, R, k, has_base, &ld, &kaug, &waug_elems, &part_elems, &span);
   const size_t need = sizeof(T) * (size_t)(waug_elems + part_elems);
   if (ws_bytes < need || (need > 0 && ws == nullptr))
     return set_error(KAN_ERR_WORKSPACE, "kan_forward: workspace of %zu bytes is smaller than the %zu required",
@@ -311,6 +381,18 @@ int forward_impl(const void* x, const void* grid, const void* bw, const void* sw
   const T* tx = static_cast<const T*>(x);
   T* taug = static_cast<T*>(aug);
   T* twaug = static_cast<T*>(ws);
+  if constexpr (std::is_same<T, float>::value) {
+    if (span.v > 0) {  // the basis is still written: the backward's parameter product reads it
+      KAN_TRY(launch_build_waug_t<T>(static_cast<const T*>(sw), static_cast<const T*>(scaler),
+                                     static_cast<const T*>(bw), twaug, kaug, O, I, R, st));
+      KAN_TRY(launch_basis<T>(tx, static_cast<const T*>(grid), taug, ld,
+                              has_base ? taug + I * R : nullptr, n, I, (int)G, (int)k,
+                              g_basis_impl.load(), st));
+      return launch_span_forward(span, tx, static_cast<const T*>(grid), twaug,
+                                 static_cast<T*>(out), twaug + waug_elems, n, I, O, (int)G, (int)k,
+                                 has_base, st);
+    }
+  }
   KAN_TRY(launch_build_waug<T>(static_cast<const T*>(sw), static_cast<const T*>(scaler),
                                static_cast<const T*>(bw), twaug, ld, O, I, R, st));
   KAN_TRY(launch_basis<T>(tx, static_cast<const T*>(grid), taug, ld,
@@ -344,6 +426,10 @@ int backward_impl(const void* D, const void* x, const void* grid, const void* bw
     KAN_TRY(launch_build_waug_t<T>(static_cast<const T*>(sw), static_cast<const T*>(scaler),
                                    static_cast<const T*>(bw), waug, p.kaug, O, I, p.R, st));
     if constexpr (std::is_same<T, float>::value) {
+      if (p.span_dx)
+        KAN_TRY(launch_span_dx(p.span, tD, static_cast<const float*>(x),
+                               static_cast<const float*>(grid), waug, static_cast<float*>(gx), E,
+                               n, I, O, (int)G, (int)k, has_base, st));
       if (p.fused_dx) {
         KAN_TRY(launch_gemm_dx(n, p.kaug, O, tD, O, waug, O, static_cast<const float*>(x),
                                static_cast<const float*>(grid), I, (int)G, (int)k, has_base, E,
@@ -364,7 +450,7 @@ int backward_impl(const void* D, const void* x, const void* grid, const void* bw
                                         static_cast<float*>(gx), n, I, (int)G, (int)k, st));
     }
   }
-  if (need_x && !p.fused_dx && !p.compact_dx) {
+  if (need_x && !p.fused_dx && !p.compact_dx && !p.span_dx) {
     // E[n, k'] = sum_o D[n, o] Waug[o, k'] = sum_o D[n, o] WaugT[k', o]  (both K-contiguous)
     KAN_TRY(launch_gemm<T>(kLayoutNT, n, p.kaug, O, tD, O, waug, O, E, p.ld, 1, 0, st));
     KAN_TRY(launch_basis_grad<T>(static_cast<const T*>(x), static_cast<const T*>(grid), E, p.ld,
@@ -762,8 +848,11 @@ int kan_hip_forward_workspace(int dtype, int64_t n, int64_t I, int64_t O, int64_
   KAN_TRY(check_layer("kan_forward_workspace", n, I, O, G, k));
   KAN_TRY(need_ptr(bytes, "kan_forward_workspace", "bytes"));
   int64_t ld, kaug, we, pe;
-  if (dtype == KAN_DTYPE_F32) forward_plan<float>(n, I, O, G + k, has_base != 0, &ld, &kaug, &we, &pe);
-  else forward_plan<double>(n, I, O, G + k, has_base != 0, &ld, &kaug, &we, &pe);
+  SpanPlan span;
+  if (dtype == KAN_DTYPE_F32)
+    forward_plan<float>(n, I, O, G + k, k, has_base != 0, &ld, &kaug, &we, &pe, &span);
+  else
+    forward_plan<double>(n, I, O, G + k, k, has_base != 0, &ld, &kaug, &we, &pe, &span);
   *bytes = (dtype == KAN_DTYPE_F32 ? 4 : 8) * (size_t)(we + pe);
   return KAN_OK;
 }
@@ -817,8 +906,9 @@ int kan_hip_infer_workspace(int dtype, int64_t n, int64_t I, int64_t O, int64_t 
   KAN_TRY(check_layer("kan_infer_workspace", n, I, O, G, k));
   KAN_TRY(need_ptr(bytes, "kan_infer_workspace", "bytes"));
   int64_t ld, kaug, a, pe;
-  if (dtype == KAN_DTYPE_F32) infer_plan<float>(n, I, O, G + k, has_base != 0, &ld, &kaug, &a, &pe);
-  else infer_plan<double>(n, I, O, G + k, has_base != 0, &ld, &kaug, &a, &pe);
+  SpanPlan span;
+  if (dtype == KAN_DTYPE_F32) infer_plan<float>(n, I, O, G + k, k, has_base != 0, &ld, &kaug, &a, &pe, &span);
+  else infer_plan<double>(n, I, O, G + k, k, has_base != 0, &ld, &kaug, &a, &pe, &span);
   *bytes = (dtype == KAN_DTYPE_F32 ? 4 : 8) * (size_t)(a + pe);
   return KAN_OK;
 }
@@ -836,12 +926,13 @@ int infer_run(int dtype, const void* x, const void* grid, const void* waug, void
   }
   const int64_t R = G + k;
   int64_t ld, kaug, aug_elems, part_elems;
+  SpanPlan span;
   const size_t elem = dtype == KAN_DTYPE_F32 ? 4 : 8;
   if (dtype == KAN_DTYPE_F32)
-    infer_plan<float>(n, I, O, R, has_base != 0, &ld, &kaug, &aug_elems, &part_elems,
+    infer_plan<float>(n, I, O, R, k, has_base != 0, &ld, &kaug, &aug_elems, &part_elems, &span,
                       scratch_elems);
   else
-    infer_plan<double>(n, I, O, R, has_base != 0, &ld, &kaug, &aug_elems, &part_elems,
+    infer_plan<double>(n, I, O, R, k, has_base != 0, &ld, &kaug, &aug_elems, &part_elems, &span,
                        scratch_elems);
   const int64_t cap = infer_slice_cap(scratch_elems, aug_elems);
   const size_t need = elem * (size_t)(aug_elems + part_elems);
@@ -849,6 +940,13 @@ int infer_run(int dtype, const void* x, const void* grid, const void* waug, void
     return set_error(KAN_ERR_WORKSPACE, "kan_infer: workspace of %zu bytes is smaller than the %zu required",
                      ws_bytes, need);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (span.v > 0) {  // fp32
+    float* wt = static_cast<float*>(ws);
+    KAN_TRY(launch_transpose(static_cast<const float*>(waug), ld, wt, O, kaug, st));
+    return launch_span_forward(span, static_cast<const float*>(x),
+                               static_cast<const float*>(grid), wt, static_cast<float*>(out),
+                               wt + aug_elems, n, I, O, (int)G, (int)k, has_base != 0, st);
+  }
 #define KAN_INFER_CALL(T)                                                                        \
   do {                                                                                           \
     T* aug = static_cast<T*>(ws);                                                                \
@@ -881,13 +979,14 @@ int kan_hip_infer_noalloc(int dtype, const void* x, const void* grid, const void
   if (n * O == 0) return KAN_OK;
   const int64_t R = G + k;
   int64_t ld, kaug, aug_elems, part_elems;
+  SpanPlan span;
   const size_t elem = dtype == KAN_DTYPE_F32 ? 4 : 8;
   const int64_t scratch_elems = (int64_t)(KAN_NOALLOC_SCRATCH_BYTES / elem);
   if (dtype == KAN_DTYPE_F32)
-    infer_plan<float>(n, I, O, R, has_base != 0, &ld, &kaug, &aug_elems, &part_elems,
+    infer_plan<float>(n, I, O, R, k, has_base != 0, &ld, &kaug, &aug_elems, &part_elems, &span,
                       scratch_elems);
   else
-    infer_plan<double>(n, I, O, R, has_base != 0, &ld, &kaug, &aug_elems, &part_elems,
+    infer_plan<double>(n, I, O, R, k, has_base != 0, &ld, &kaug, &aug_elems, &part_elems, &span,
                        scratch_elems);
   const size_t need = elem * (size_t)(aug_elems + part_elems);
   if (need > (size_t)KAN_NOALLOC_SCRATCH_BYTES)

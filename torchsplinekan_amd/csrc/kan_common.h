@@ -250,6 +250,30 @@ int launch_matmul(int layout, int64_t M, int64_t N, int64_t K, const T* A, int64
 template <typename T>
 int gemm_pick_splits(int64_t M, int64_t N, int64_t K, int64_t max_slice_elems = -1);
 
+// Estimated seconds of an fp32 product M x N x K as launch_matmul runs it.
+double gemm_seconds_f32(int64_t M, int64_t N, int64_t K);
+
+// Span-window products of a layer with many basis functions per feature
+// (kan_span.hip): y and dx from x, the knots and the transposed augmented
+// weight wt [kaug, O], without the basis or E.  part holds plan.part_elems.
+struct SpanPlan {
+  int v;                            // outputs per lane
+  int64_t tiles_n, tiles_o, slices;
+  int64_t feats;                    // features per slice
+  int64_t part_elems;
+  double seconds;                   // estimate
+};
+SpanPlan span_plan(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, bool dx);
+int launch_span_forward(const SpanPlan& pl, const float* x, const float* grid, const float* wt,
+                        float* y, float* part, int64_t n, int64_t I, int64_t O, int G, int k,
+                        bool base, hipStream_t st);
+int launch_span_dx(const SpanPlan& pl, const float* D, const float* x, const float* grid,
+                   const float* wt, float* gx, float* part, int64_t n, int64_t I, int64_t O, int G,
+                   int k, bool base, hipStream_t st);
+// wt [kaug, O] = the transpose of w's first kaug columns (rows of ld).
+int launch_transpose(const float* w, int64_t ld, float* wt, int64_t O, int64_t kaug,
+                     hipStream_t st);
+
 // fp64 edge statistic on MFMA (kan_edge_mfma64.hip), for R + 1 <= 16; the
 // VALU kernels of kan_edge.hip serve wider rows.
 bool edge_mfma64_applies(int64_t R);

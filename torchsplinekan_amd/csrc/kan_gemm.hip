@@ -1981,6 +1981,14 @@ int gemm_pick_splits(int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
   return best;
 }
 
+double gemm_seconds_f32(int64_t M, int64_t N, int64_t K) {
+  if (gemm_is_thin(M, N, K))  // bound by its largest operand
+    return 4.0 * (double)std::max({M * N, M * K, N * K}) / 2e12;
+  const int64_t cus = device_cu_count();
+  const int s = gemm_pick_splits<float>(M, N, K, -1);
+  return est_seconds(kModelF32[pick_cfg_f32(M, N, K, s, cus)], M, N, K, s, cus);
+}
+
 template <typename T>
 int launch_gemm(int layout, int64_t M, int64_t N, int64_t K, const T* A, int64_t lda, const T* B,
                 int64_t ldb, T* C, int64_t ldc, int splits, int64_t split_stride,

@@ -100,3 +100,31 @@ def test_span_inputs_and_weights_that_are_not_finite():
     assert torch.equal(y == float("inf"), want == float("inf"))
     ok = want.isfinite()
     assert _norm(y[ok], want[ok].double()) < 1e-5
+
+
+def test_span_products_in_a_captured_graph():
+    n, I, O, G, k, base = shape = (4729, 948, 61, 65, 3, True)
+    assert all(_routes(*shape))
+    x, grid, bw, sw, sc = _layer(*shape)
+    D = torch.randn(n, O, device="cuda")
+    xg = x.clone().requires_grad_()
+
+    def step():
+        y = _C.kan_apply(xg, grid, bw, sw, sc, k, True)
+        return y, torch.autograd.grad(y, xg, D)[0]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y, dx = step()
+    for seed in (3, 4):
+        with torch.no_grad():
+            xg.copy_(_layer(*shape, seed=seed)[0])
+        graph.replay()
+        ey, edx = step()
+        assert torch.equal(y, ey) and torch.equal(dx, edx)

@@ -81,3 +81,14 @@ def test_error_has_no_mean():
         err = _C.matmul(A.cuda(), B.cuda()).cpu().double() - A.double() @ B.double()
     limit = 5 * float(err.std()) / (M * N) ** 0.5 + 0.01 * 3e-8 * (K / 16)
     assert abs(float(err.mean())) < limit
+
+
+def test_leading_dimension_past_a_buffer_resource():
+    """256 rows of 2.2 million columns span more than 2^31 bytes: the loads
+    with 64-bit addresses."""
+    M, N, K = 300, 70, 150
+    wide = torch.empty(M, 2_200_000, device="cuda")
+    A, B = _operands(M, N, K, False, True, seed=5)
+    wide[:, :K] = A.cuda()
+    got = _C.matmul(wide[:, :K], B.cuda())
+    assert torch.equal(got, _C.matmul(A.cuda(), B.cuda()))

@@ -203,3 +203,18 @@ def test_c_header_compiles_as_c(tmp_path):
                         "-c", str(src), "-o", str(tmp_path / "t.o")], capture_output=True,
                        text=True)
     assert r.returncode == 0, r.stderr
+
+
+@pytest.mark.parametrize("n,O", [(1920, 8_020_000), (1920, 4_194_241), (100_000, 8_020_001)])
+def test_inference_of_very_many_outputs_keeps_64_bit_offsets(lib, n, O):
+    """The span-window kernels address a feature's R rows of the transposed
+    weight with 32-bit offsets (R O 4 bytes, 2^31 at O = 7.9 million), and its
+    transpose takes 65535 blocks of 64 outputs: wider layers stay on the dense
+    product (the workspace tells the two routes apart)."""
+    def workspace():
+        nbytes = ctypes.c_size_t(0)
+        lib.check(lib.LIB.kan_hip_infer_workspace(0, n, 8, O, 65, 3, 1, ctypes.byref(nbytes)))
+        return nbytes.value
+    auto = workspace()
+    with lib.route("compact_e", 1):      # the dense product
+        assert auto == workspace()

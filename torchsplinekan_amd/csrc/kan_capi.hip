@@ -231,8 +231,13 @@ int need_ptr(const void* p, const char* who, const char* name) {
 // than the dense product, which costs R + 1 columns a feature where they cost
 // k + 2.
 constexpr int64_t kSpanMinR = 40;
+// The transposed weight's launch holds 65535 blocks of 64 outputs, and up to
+// there a feature's R rows of it (R O 4 bytes) lie within the span kernels'
+// 32-bit buffer offsets; wider layers take the dense product's 64-bit ones.
+constexpr int64_t kSpanMaxO = 65535 * 64;
+static_assert(kMaxR * kSpanMaxO * 4 < (int64_t)1 << 31, "a feature's rows within a buffer resource");
 bool span_may(int64_t n, int64_t I, int64_t O, int64_t R) {
-  return R >= kSpanMinR && n > 0 && I > 0 && O > 0 && g_basis_impl.load() == 1 &&
+  return R >= kSpanMinR && O <= kSpanMaxO && n > 0 && I > 0 && O > 0 && g_basis_impl.load() == 1 &&
          kan_hip_get_route(KAN_ROUTE_COMPACT_E) == -1 &&
          kan_hip_get_route(KAN_ROUTE_FUSED_DX) == 0 &&
          kan_hip_get_route(KAN_ROUTE_GEMM_TILE) == -1;

@@ -82,24 +82,35 @@ def test_span_products_match_float64(shape):
     assert torch.equal(yi, _C.kan_infer(x, grid, waug, k, base))    # fixed order of sums
 
 
+def _same_classes(y, want):
+    """NaN and infinities in the same places (sign included), the rest close."""
+    assert torch.equal(y.isnan(), want.isnan())
+    assert torch.equal(y.isinf(), want.isinf())
+    assert torch.equal(y[y.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    assert _norm(y[ok], want[ok].double()) < 1e-5
+
+
 def test_span_inputs_and_weights_that_are_not_finite():
     """As in the dense product: NaN or infinite inputs reach their row through
-    silu alone; a weight that is not finite reaches its output's every sample."""
+    silu alone; a weight that is not finite reaches its output's every sample,
+    times the sample's basis value or silu, or times zero."""
     shape = (3000, 333, 61, 66, 2, True)
     assert _routes(*shape)[0]
     x, grid, bw, sw, sc = _layer(*shape)
     bw = bw.abs() + 0.1
-    x[5, 7], x[6, 8], x[7, 9] = float("nan"), float("inf"), 50.0
+    x[5, 7], x[6, 8], x[7, 9], x[8, 10], x[9, 50] = float("nan"), float("inf"), 50.0, 0.0, -50.0
     sw[3, 100, 20] = float("nan")
+    sw[5, 50, 30], sw[6, 50, 0], sw[7, 332, 67] = float("inf"), -float("inf"), float("inf")
+    bw[8, 10], bw[9, 11] = float("inf"), -float("inf")
     waug = _C.pack_weight(bw, sw, sc, 2, True)
     y = _C.kan_infer(x, grid, waug, 2, True)
     with _lib.route("compact_e", 1):     # the dense product
         want = _C.kan_infer(x, grid, waug, 2, True)
-    assert torch.equal(y.isnan(), want.isnan()) and bool(y[5].isnan().all())
-    assert bool(y[:, 3].isnan().all())
-    assert torch.equal(y == float("inf"), want == float("inf"))
-    ok = want.isfinite()
-    assert _norm(y[ok], want[ok].double()) < 1e-5
+    assert bool(y[5].isnan().all()) and bool(y[:, 3].isnan().all())
+    for o in (5, 8, 9):                  # infinities among them
+        assert bool(want[:, o].isinf().any()) and not bool(want[:, o].isfinite().any())
+    _same_classes(y, want)
 
 
 def test_span_products_in_a_captured_graph():

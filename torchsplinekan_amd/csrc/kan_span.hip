@@ -159,15 +159,12 @@ span_kernel(SpanParams p) {
     }
     if (r0 == 0) *reinterpret_cast<u32x4*>(buf + (R + 2 * K) * OB + 4 * cg) = sb;
     if constexpr (!DX) {
-      // (a weight that is not finite reaches every sample, as 0 times it does
-      // in the dense product)
+      // (NaN where a spline weight is not finite: see the end)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int u = 0; u < kLoads; ++u)
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u)
+        for (int j = 0; j < 4; ++j)
           poison[j] = __builtin_fmaf(__uint_as_float(st[u][j]), 0.0f, poison[j]);
-        poison[j] = __builtin_fmaf(__uint_as_float(sb[j]), 0.0f, poison[j]);
-      }
     }
   };
 
@@ -319,16 +316,43 @@ span_kernel(SpanParams p) {
     }
   }
   if constexpr (!DX) {
-    // 0, or NaN where a weight of the slice's features was not finite
+    // A spline weight that is not finite meets every sample in the dense
+    // product: times a basis value where the sample's window holds it (the
+    // loop above), times 0 elsewhere.  A block that staged one adds these
+    // zeros' products here, so that infinities and NaN come out as they do
+    // there.  (The base weights met every sample above.)
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < 4; ++j) lds[r0 * OB + 4 * cg + j] = poison[j];
     __syncthreads();
-    float add[V];
+    float any = 0.0f;
 #pragma unroll
-    for (int v = 0; v < V; ++v) {
-      add[v] = 0.0f;
-      for (int r = 0; r < kRowsPer; ++r) add[v] += lds[r * OB + lane * V + v];
+    for (int v = 0; v < V; ++v)
+      for (int r = 0; r < kRowsPer; ++r) any += lds[r * OB + lane * V + v];
+    if (__any(any != 0.0f)) {
+#pragma unroll 1
+      for (int64_t f = fbeg; f < fend; ++f) {
+        const int m = knot_span(p.grid + f * nk, nk, p.x[ns * p.I + f]);
+#pragma unroll 1
+        for (int r = 0; r < R; ++r) {
+          float z[V];  // 0, or NaN
+          bool bad = false;
+#pragma unroll
+          for (int v = 0; v < V; ++v) {
+            const int64_t o = o0 + lane * V + v;
+            z[v] = o < p.O ? p.wt[(f * R + r) * p.O + o] * 0.0f : 0.0f;
+            bad |= z[v] != 0.0f;
+          }
+          if (!__any(bad)) continue;
+#pragma unroll
+          for (int s = 0; s < kSpanS; ++s) {
+            const int ms = __builtin_amdgcn_readlane(m, s);
+            if (ms >= 0 && r >= ms - K && r <= ms) continue;
+#pragma unroll
+            for (int v = 0; v < V; ++v) blk[s][v] += z[v];
+          }
+        }
+      }
     }
     float* out = p.out + (int64_t)slice * p.out_stride;
 #pragma unroll
@@ -337,7 +361,7 @@ span_kernel(SpanParams p) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const int64_t o = o0 + lane * V + v;
-        if (o < p.O) out[(n0 + s) * p.O + o] = blk[s][v] + add[v];
+        if (o < p.O) out[(n0 + s) * p.O + o] = blk[s][v];
       }
     }
   }

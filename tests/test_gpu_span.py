@@ -113,6 +113,39 @@ def test_span_inputs_and_weights_that_are_not_finite():
     _same_classes(y, want)
 
 
+@pytest.mark.parametrize("shape", [(4500, 500, 61, 65, 2, False), (4729, 948, 61, 65, 3, True),
+                                   (4500, 500, 256, 65, 3, True),
+                                   (1281, 1068, 461, 65, 1, True)])
+def test_span_input_gradient_of_values_that_are_not_finite(shape):
+    """As from the dense product's window rows: an x outside the knots meets
+    no spline weight and, without a base branch, no dL/dy."""
+    n, I, O, G, k, base = shape
+    assert _routes(*shape)[1]
+    x, grid, bw, sw, sc = _layer(*shape)
+    D = torch.randn(n, O, generator=torch.Generator().manual_seed(1)).cuda()
+    x[0:3] = 40.0                        # outside every feature's knots
+    x[3, 5], x[4, 6], x[5, 7] = float("nan"), float("inf"), -float("inf")
+    inf = float("inf")
+    D[0, 3], D[10, 4], D[11, 5], D[12, 6], D[12, 9] = inf, inf, -inf, inf, -inf
+    D[1, 2], D[13, 7] = float("nan"), float("nan")
+    sw[3, 20, 0], sw[4, 21, 1], sw[5, 22, 30] = float("nan"), inf, -inf
+    sw[O - 1, I - 1, G + k - 1] = inf
+    if base:
+        bw[2, 30], bw[3, 31] = inf, float("nan")
+
+    def dx():
+        xg = x.clone().requires_grad_()
+        return torch.autograd.grad(_C.kan_apply(xg, grid, bw, sw, sc, k, True), xg, D)[0]
+
+    got = dx()
+    with _lib.route("compact_e", 1):     # the dense product and its windows
+        want = dx()
+    if not base:
+        assert torch.equal(got[0:3], torch.zeros_like(got[0:3]))
+    assert bool(want.isinf().any()) and bool(want.isnan().any())
+    _same_classes(got, want)
+
+
 def test_span_products_in_a_captured_graph():
     n, I, O, G, k, base = shape = (4729, 948, 61, 65, 3, True)
     assert all(_routes(*shape))

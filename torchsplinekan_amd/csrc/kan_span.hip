@@ -400,6 +400,63 @@ __global__ void span_sum_kernel(const float* __restrict__ part, int slices, int6
   }
 }
 
+// The input gradient's items that came out infinite or NaN, evaluated again in
+// the dense product's order: each weight row of the item's window summed over
+// the outputs, then times its derivative.  The span kernel's sums differ there
+// (0 times such a value, the rows it reads for an x outside the knots,
+// infinities of both signs).  A wave looks through 256 items at a time and
+// takes a bad one with all its lanes; where there is none the pass costs its
+// reads (a kernel of its own, since the span kernel has no register left: the
+// same check at its end took 3 % of it, the pass takes 1 %).
+constexpr int kAgainItems = 4;  // per lane
+template <int K>
+__global__ __launch_bounds__(256) void span_dx_again_kernel(SpanParams p, float* __restrict__ gx) {
+  const int lane = threadIdx.x & 63;
+  const int64_t count = p.n * p.I, step = (int64_t)gridDim.x * 256 * kAgainItems;
+  const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64 * kAgainItems;
+#pragma unroll 1
+  for (int64_t e0 = first; e0 < count; e0 += step) {
+    float v[kAgainItems];
+#pragma unroll
+    for (int u = 0; u < kAgainItems; ++u) {
+      const int64_t e = e0 + 64 * u + lane;
+      v[u] = e < count ? gx[e] : 0.0f;
+    }
+#pragma unroll 1
+    for (int u = 0; u < kAgainItems; ++u) {
+      uint64_t again = __ballot(v[0] * 0.0f != 0.0f);
+#pragma unroll
+      for (int w = 0; w + 1 < kAgainItems; ++w) v[w] = v[w + 1];
+#pragma unroll 1
+      for (; again != 0; again &= again - 1) {
+        const int64_t e = e0 + 64 * u + __builtin_ctzll(again);
+        const int64_t n = e / p.I, f = e - n * p.I;
+        const float* tk = p.grid + f * p.nk;
+        const float xv = p.x[e];
+        const int m = knot_span(tk, p.nk, xv);
+        float b[K + 1];
+        span_derivs<K, float>(tk, p.nk, m >= 0 ? m : K, xv, b);
+        auto row_sum = [&](int64_t row) {
+          float a = 0.0f;
+          for (int64_t o = lane; o < p.O; o += 64)
+            a = __builtin_fmaf(p.D[n * p.O + o], p.wt[row * p.O + o], a);
+#pragma unroll
+          for (int off = 32; off >= 1; off >>= 1) a += __shfl_xor(a, off);
+          return a;
+        };
+        float q = 0.0f;
+#pragma unroll
+        for (int j = 0; j <= K; ++j) {
+          const int r = m - K + j;
+          if (m >= 0 && r >= 0 && r < p.R) q += row_sum(f * p.R + r) * b[j];
+        }
+        if (p.base) q += row_sum(p.I * p.R + f) * silu_grad_of<float>(xv);
+        if (lane == 0) gx[e] = q;
+      }
+    }
+  }
+}
+
 size_t span_lds_bytes(int K, int V, int R, int nk) {
   const size_t need = sizeof(float) * (2 * (size_t)(R + 2 * K + 1) * 64 * V + 4 * (size_t)nk);
   return std::max(need, sizeof(float) * 4 * (size_t)kSpanThreads);  // (the poison's reduction)
@@ -547,7 +604,16 @@ int launch_span_dx(const SpanPlan& pl, const float* D, const float* x, const flo
     const int rc = launch_span<true>(p, k, pl.v, st);
     if (rc != KAN_OK) return rc;
   }
-  return pl.tiles_o > 1 ? sum_parts(part, pl.tiles_o, n * I, gx, st) : KAN_OK;
+  if (pl.tiles_o > 1) {
+    const int rc = sum_parts(part, pl.tiles_o, n * I, gx, st);
+    if (rc != KAN_OK) return rc;
+  }
+  TimedLaunch timed(kClassOther, st, 0.0);
+  const dim3 blocks((unsigned)std::min<int64_t>(ceil_div(n * I, (int64_t)(256 * kAgainItems)), 4096));
+  if (k == 1) hipLaunchKernelGGL(span_dx_again_kernel<1>, blocks, dim3(256), 0, st, p, gx);
+  else if (k == 2) hipLaunchKernelGGL(span_dx_again_kernel<2>, blocks, dim3(256), 0, st, p, gx);
+  else hipLaunchKernelGGL(span_dx_again_kernel<3>, blocks, dim3(256), 0, st, p, gx);
+  return check_launch("span input gradient, values that are not finite");
 }
 
 int launch_transpose(const float* w, int64_t ld, float* wt, int64_t O, int64_t kaug,

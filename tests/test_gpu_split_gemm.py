@@ -69,6 +69,19 @@ def test_non_finite_and_overflowing_values(tile, ta, tb):
     assert bool((err <= (K + 8) * 2.0 ** -24 * (A[rest].double().abs() @ B.double().abs())).all())
 
 
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("K", [40, 256, 257, 400, 513, 1000])
+def test_zero_sums_are_positive(tile, K):
+    """Rows of zeros give +0, whichever sign the sums end with (outputs large
+    enough that K is not split)."""
+    M, N = 2304, 64 if tile == "256x64" else 2304
+    A, B = _operands(M, N, K, False, True, seed=K)
+    A[::2] = 0.0
+    with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+        got = _C.matmul(A.cuda(), B.cuda())[::2]
+    assert not bool(got.any()) and not bool(got.signbit().any())
+
+
 def test_error_has_no_mean():
     """The MFMA's rounding towards minus infinity must not add up: over 65536
     output values the mean error lies within five standard errors plus a

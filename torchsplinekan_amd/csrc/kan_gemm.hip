@@ -297,12 +297,19 @@ __device__ __forceinline__ void read_frag_il(const T* __restrict__ lds, int row0
   }
 }
 
+// An fp32 tile's sums hold its values times 1 / back, 1 or -1 (scaled_back
+// gives +0 for a zero of either sign).
+__device__ __forceinline__ float scaled_back(float v, float back) {
+  return __builtin_fmaf(v, back, 0.0f);
+}
+
 // Writes the wave's accumulators to C (+ split slice), bounds-checked.  AIL /
 // BIL: the rows / columns of the MFMA tiles are interleaved (read_frag_il).
+// back: see scaled_back (fp32).
 template <class C, typename Acc, bool AIL = false, bool BIL = false>
 __device__ __forceinline__ void store_tile(const GemmParams<typename C::T>& p, const TileCoords& tc,
                                            const Acc (&acc)[C::FM][C::FN], int wm, int wn,
-                                           int lane) {
+                                           int lane, float back = 1.0f) {
   typedef Mfma<typename C::T, C::MF> M;
   typename C::T* Cp = p.C + (int64_t)tc.split * p.split_stride;
 #pragma unroll
@@ -316,7 +323,11 @@ __device__ __forceinline__ void store_tile(const GemmParams<typename C::T>& p, c
       for (int v = 0; v < M::kNAcc; ++v) {
         const int rl = M::out_row(lane, v);
         const int64_t row = tc.m0 + wm * C::TM + (AIL ? C::FM * rl + i : i * C::MF + rl);
-        if (row < p.M) Cp[row * p.ldc + col] = acc[i][j][v];
+        if (row >= p.M) continue;
+        if constexpr (std::is_same<typename C::T, float>::value)
+          Cp[row * p.ldc + col] = scaled_back(acc[i][j][v], back);
+        else
+          Cp[row * p.ldc + col] = acc[i][j][v];
       }
     }
   }
@@ -513,9 +524,9 @@ __device__ __forceinline__ int div_small(int v, float rcp) {
 template <class C, int K>
 __device__ __forceinline__ void dx_epilogue(const GemmParams<float>& p, const DxParams& e,
                                             const TileCoords& tc,
-                                            const f32x16 (&acc)[C::FM][C::FN], float* lds_stage,
-                                            float* lds_side, int side_floats, int wave, int wm,
-                                            int wn, int lane) {
+                                            const f32x16 (&acc)[C::FM][C::FN], float back,
+                                            float* lds_stage, float* lds_side, int side_floats,
+                                            int wave, int wm, int wn, int lane) {
   typedef Mfma<float, 32> M;
   constexpr int TN = C::TN, SW = C::TN + 1;  // staged row stride (odd: conflict-free columns)
   float* stage = lds_stage + wave * 32 * SW;
@@ -572,7 +583,8 @@ __device__ __forceinline__ void dx_epilogue(const GemmParams<float>& p, const Dx
     for (int j = 0; j < C::FN; ++j)
 #pragma unroll
       for (int v = 0; v < M::kNAcc; ++v)
-        stage[M::out_row(lane, v) * SW + j * 32 + M::out_col(lane)] = acc[iq][j][v];
+        stage[M::out_row(lane, v) * SW + j * 32 + M::out_col(lane)] =
+            scaled_back(acc[iq][j][v], back);
     wave_sync_lds();
     const float* xq = xs + (iq - q0) * 32 * per_row;
     // items (sample row, idx) of this tile row, idx fastest across lanes
@@ -632,7 +644,7 @@ __device__ __forceinline__ void dx_epilogue(const GemmParams<float>& p, const Dx
 template <class C, int K>
 __device__ __forceinline__ void ecomp_epilogue(const GemmParams<float>& p, const DxParams& e,
                                                const TileCoords& tc,
-                                               const f32x16 (&acc)[C::FM][C::FN],
+                                               const f32x16 (&acc)[C::FM][C::FN], float back,
                                                float* lds_stage, float* lds_side, int side_floats,
                                                int wave, int wm, int wn, int lane) {
   typedef Mfma<float, 32> M;
@@ -649,7 +661,7 @@ __device__ __forceinline__ void ecomp_epilogue(const GemmParams<float>& p, const
 #pragma unroll
         for (int v = 0; v < M::kNAcc; ++v) {
           const int64_t row = tc.m0 + (int64_t)wm * C::TM + iq * 32 + M::out_row(lane, v);
-          if (row < p.M) e.es[row * e.I + (col - e.ksp)] = acc[iq][j][v];
+          if (row < p.M) e.es[row * e.I + (col - e.ksp)] = scaled_back(acc[iq][j][v], back);
         }
       }
   }
@@ -722,7 +734,8 @@ __device__ __forceinline__ void ecomp_epilogue(const GemmParams<float>& p, const
     for (int j = 0; j < C::FN; ++j)
 #pragma unroll
       for (int v = 0; v < M::kNAcc; ++v)
-        stage[M::out_row(lane, v) * SW + j * 32 + M::out_col(lane)] = acc[iq][j][v];
+        stage[M::out_row(lane, v) * SW + j * 32 + M::out_col(lane)] =
+            scaled_back(acc[iq][j][v], back);
     wave_sync_lds();
     const float* sq = xs + (iq - q0) * 32 * nfs;
     for (int it = lane; it < 32 * nfs; it += 64) {
@@ -1115,6 +1128,7 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  float back = 1.0f;
   // body: the load mode of every slab but the last, tail: the last one's
   auto run = [&](auto body_c, auto tail_c) KAN_INLINE_LAMBDA {
     if (tc.nkt > 1) {
@@ -1154,7 +1168,7 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
     }
     slab(kt, IC<0>(), IC<0>(), tail_c);
     acc[FM - 1][FN - 1] += tmp[1];
-    if (turned(kt)) negate();
+    if (turned(kt)) back = -back;
   };
   if (tc.nkt > 0) {
     if (p.buf) run(IC<1>(), IC<2>());
@@ -1176,11 +1190,13 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
   int bad = 0;
 #pragma unroll
   for (int w = 0; w < C::WM * C::WN; ++w) bad |= flags[w];
-  if (__builtin_amdgcn_readfirstlane(bad) != 0)
+  if (__builtin_amdgcn_readfirstlane(bad) != 0) {
     fp32_tile<C, AK, BKC>(p, tc, acc, reinterpret_cast<float*>(lds), wm, wn, lane);
+    back = 1.0f;
+  }
   if constexpr (EPIK == 0) {
     (void)e;
-    store_tile<C, f32x16>(p, tc, acc, wm, wn, lane);
+    store_tile<C, f32x16>(p, tc, acc, wm, wn, lane, back);
   } else {
     float* stage = reinterpret_cast<float*>(lds);
     float* side = reinterpret_cast<float*>(lds + Lds::kStage);
@@ -1188,9 +1204,9 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
     static_assert(kSide + 512 <= 8192, "div_small covers the side buffer's indices");
     __syncthreads();  // every wave has read the flags
     if constexpr (EPIK > 0)
-      dx_epilogue<C, EPIK>(p, e, tc, acc, stage, side, kSide, wave, wm, wn, lane);
+      dx_epilogue<C, EPIK>(p, e, tc, acc, back, stage, side, kSide, wave, wm, wn, lane);
     else
-      ecomp_epilogue<C, -EPIK>(p, e, tc, acc, stage, side, kSide, wave, wm, wn, lane);
+      ecomp_epilogue<C, -EPIK>(p, e, tc, acc, back, stage, side, kSide, wave, wm, wn, lane);
   }
 }
 

@@ -70,6 +70,43 @@ def test_non_finite_and_overflowing_values(tile, ta, tb):
 
 
 @pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("power", [-109, -112, -120, -128, -140, -146])
+def test_operands_below_the_split_parts(tile, ta, tb, power):
+    """An operand below 2^-110 would have low parts past bf16's last bit 2^-133
+    (none left at 2^-134); with a large other operand its products are
+    ordinary numbers, and they keep fp32's accuracy: as whole operands, and as
+    one value, in the first or the last slab."""
+    M, N, K = 70, 40, 100
+    A, B = _operands(M, N, K, ta, tb, seed=-power)
+    small = (A.double() * 2.0 ** power).float()
+    with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+        _check(small, B * 2.0 ** 60)
+        _check(A * 2.0 ** 60, (B.double() * 2.0 ** power).float())
+        for k in (3, K - 1):
+            one = A.clone()
+            one[9], B2 = 0.0, B.clone()
+            one[9, k] = small[9, k]
+            B2[k] = B[k] * 2.0 ** 60
+            got = _C.matmul(one.cuda(), B2.cuda())[9].cpu().double()
+            want = small[9, k].double() * B2[k].double()
+            # one product: the last MFMA truncates (2^-23), the five before it at
+            # 2^-8 of that or less, the dropped parts 2^-26
+            assert bool(((got - want).abs() <= 1.25 * 2.0 ** -23 * want.abs()).all())
+
+
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+@pytest.mark.parametrize("pa,pb", [(-64, -60), (46, 45), (100, 18), (18, 100), (115, 3), (126, -40)])
+def test_small_and_large_products(tile, ta, tb, pa, pb):
+    """Products near both ends of fp32's range (those whose scaled sums or
+    parts overflow are evaluated in plain fp32)."""
+    A, B = _operands(70, 40, 100, ta, tb, seed=pa)
+    with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+        _check(A.clamp(-1.9, 1.9) * 2.0 ** pa, B * 2.0 ** pb)
+
+
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
 @pytest.mark.parametrize("K", [40, 256, 257, 400, 513, 1000])
 def test_zero_sums_are_positive(tile, K):
     """Rows of zeros give +0, whichever sign the sums end with (outputs large

@@ -297,8 +297,8 @@ __device__ __forceinline__ void read_frag_il(const T* __restrict__ lds, int row0
   }
 }
 
-// An fp32 tile's sums hold its values times 1 / back, 1 or -1 (scaled_back
-// gives +0 for a zero of either sign).
+// An fp32 tile's sums hold its values times 1 / back (scaled_back gives +0
+// for a zero of either sign).
 __device__ __forceinline__ float scaled_back(float v, float back) {
   return __builtin_fmaf(v, back, 0.0f);
 }
@@ -766,9 +766,14 @@ struct EpiSide {
 
 // ---- fp32 on bf16 MFMA: three-way split operands ---------------------------
 //
-// An fp32 value is the sum of three bf16 values, x = hi + mid + lo, exactly
-// (8 significant bits each, every part rounded to nearest, so mid <= 2^-9 |x|
-// and lo <= 2^-18 |x|).  A product of two such sums needs six bf16 products
+// An fp32 value times 2^24 is the sum of three bf16 values, hi + mid + lo,
+// exactly (8 significant bits each, every part rounded to nearest, so mid <=
+// 2^-9 and lo <= 2^-18 of it).  The factor takes fp32's last bit, 2^-149, to
+// 2^-125, so that no part is a subnormal bf16 value: without it an operand
+// below 2^-110 lost its low parts (1e-37 times 1e30 came out 5e-4 off).  It stands where A's sign is set anyhow, so B
+// alone pays for it, one VALU operation a value (forward 65536 x 1024 x 14336
+// 8.78 -> 8.90 ms, input-side and parameter products within 1 %, 5003 x 77 x
+// 3311 54 -> 57 us); the sums are scaled back as they are stored.  A product of two such sums needs six bf16 products
 // to fp32 accuracy (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three
 // dropped ones are below 2^-26 of the product.  Every product of two bf16
 // values is exact in fp32 and the MFMA accumulates in fp32, so the result
@@ -803,9 +808,9 @@ struct EpiSide {
 // K % 16 != 0: 0.143 -> 0.055 ms.
 //
 // Layout: operands are split on their way from registers to LDS (5.5 VALU
-// operations a value, hidden behind the MFMAs), so global memory holds fp32
-// only and either global layout becomes the K-contiguous rows the MFMA reads
-// with 16-byte loads.  Slabs are one MFMA deep (16 k; 48 KB for 256 + 256
+// operations a value and one to scale it, hidden behind the MFMAs), so global
+// memory holds fp32 only and either global layout becomes the K-contiguous
+// rows the MFMA reads with 16-byte loads.  Slabs are one MFMA deep (16 k; 48 KB for 256 + 256
 // rows) and double buffered.  Per slab a wave keeps B's fragments and two
 // rows of A's; a slab's stores, the loads of the slab after next and the
 // adds are spread over its tiles, and the barrier that publishes the next
@@ -822,6 +827,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitBK = 16;        // k depth of a slab: one 32x32x16 MFMA
 constexpr int kSplitRowBytes = 32;  // 16 bf16 values of one plane
 constexpr int kSplitRun = 16;       // slabs between sign changes (a power of two)
+constexpr float kSplitScale = 16777216.0f;  // of the values that are split: 2^24
 
 __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2){a, b}, bf16x2));
@@ -922,15 +928,14 @@ struct SplitLoader {
     }
   }
 
-  // The values times -1 where flip is the sign bit (0: as they are).
-  __device__ __forceinline__ void store(char* __restrict__ lds, uint32_t flip) const {
+  // The values times scale (kSplitScale, or less than zero of it).
+  __device__ __forceinline__ void store(char* __restrict__ lds, float scale) const {
 #pragma unroll
     for (int p = 0; p < kPer; ++p) {
       u32x4 hi, mid, lo;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float x0 = __uint_as_float(__float_as_uint(reg[p][2 * j]) ^ flip);
-        const float x1 = __uint_as_float(__float_as_uint(reg[p][2 * j + 1]) ^ flip);
+        const float x0 = reg[p][2 * j] * scale, x1 = reg[p][2 * j + 1] * scale;
         const unsigned int h = pack_bf16(x0, x1);
         const float r0 = x0 - bf16_lo(h), r1 = x1 - bf16_hi(h);
         const unsigned int m = pack_bf16(r0, r1);
@@ -948,10 +953,11 @@ struct SplitLoader {
 
 // The same tile in plain fp32 (v_mfma_f32_32x32x2f32, guarded loads, one
 // slab at a time): the result where a split product is not finite.  A part
-// of an infinite or nearly overflowing value times a part of the opposite
-// sign gives NaN or infinity where the fp32 product has a value, so a block
-// that meets a non-finite sum evaluates its tile again here, and what the
-// caller sees is the fp32 arithmetic's infinity, NaN or number.
+// of an infinite or large value (2^103 on) times a part of the opposite sign
+// gives NaN or infinity where the fp32 product has a value, and a scaled sum
+// overflows from 2^79 on, so a block that meets a non-finite sum evaluates
+// its tile again here, and what the caller sees is the fp32 arithmetic's
+// infinity, NaN or number.
 template <class C, bool AK, bool BKC>
 __device__ __forceinline__ void fp32_tile(const GemmParams<float>& p, const TileCoords& tc,
                                           f32x16 (&acc)[C::FM][C::FN], float* lds, int wm, int wn,
@@ -1116,11 +1122,11 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
         read_b(nxt, 0);
       }
       if (STORE && t == 0) {
-        la.store(nxt, (uint32_t)turned(kt + 1) << 31);
+        la.store(nxt, turned(kt + 1) ? -kSplitScale : kSplitScale);
         if (LOAD) gload_a(kt + 2, full_c);
       }
       if (STORE && t == kTiles / 2) {
-        lb.store(nxt + 3 * LA::kPlane, 0);
+        lb.store(nxt + 3 * LA::kPlane, kSplitScale);
         if (LOAD) gload_b(kt + 2, full_c);
       }
       tmp[t & 1] = product(af[i & 1], bf[j]);
@@ -1128,7 +1134,7 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  float back = 1.0f;
+  float back = 1.0f / (kSplitScale * kSplitScale);
   // body: the load mode of every slab but the last, tail: the last one's
   auto run = [&](auto body_c, auto tail_c) KAN_INLINE_LAMBDA {
     if (tc.nkt > 1) {
@@ -1138,8 +1144,8 @@ gemm_split_kernel(GemmParams<float> p, DxParams e) {
       gload_a(0, tail_c);
       gload_b(0, tail_c);
     }
-    la.store(lds, (uint32_t)turned(0) << 31);
-    lb.store(lds + 3 * LA::kPlane, 0);
+    la.store(lds, turned(0) ? -kSplitScale : kSplitScale);
+    lb.store(lds + 3 * LA::kPlane, kSplitScale);
     if (tc.nkt > 2) {
       gload_a(1, body_c);
       gload_b(1, body_c);

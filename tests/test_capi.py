@@ -218,3 +218,16 @@ def test_inference_of_very_many_outputs_keeps_64_bit_offsets(lib, n, O):
     auto = workspace()
     with lib.route("compact_e", 1):      # the dense product
         assert auto == workspace()
+
+
+@pytest.mark.parametrize("trans,M,N,K,limit", [
+    ((1, 0), 1024, 14336, 65536, 8192), ((1, 0), 1024, 14336, 16384, 8192),
+    ((1, 0), 1024, 14336, 8193, 8192), ((1, 0), 469, 32130, 41700, 8192),
+    ((0, 1), 65536, 1024, 16385, 16384), ((0, 1), 20000, 1300, 66600, 16384),
+    ((0, 0), 20000, 1300, 40000, 16384)])
+def test_long_fp32_sums_are_split(lib, trans, M, N, K, limit):
+    """A chain of fp32 sums is at most 8192 samples or 16384 columns long,
+    also where one slice would fill the chip."""
+    nbytes = ctypes.c_size_t(0)
+    lib.check(lib.LIB.kan_hip_matmul_workspace(0, *trans, M, N, K, ctypes.byref(nbytes)))
+    assert nbytes.value // (4 * M * N) * limit >= K

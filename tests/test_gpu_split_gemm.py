@@ -142,3 +142,20 @@ def test_leading_dimension_past_a_buffer_resource():
     wide[:, :K] = A.cuda()
     got = _C.matmul(wide[:, :K], B.cuda())
     assert torch.equal(got, _C.matmul(A.cuda(), B.cuda()))
+
+
+def test_long_sums_of_samples():
+    """A parameter product of 65536 samples with a mean, large enough to fill
+    the chip unsplit.  A running sum rounds once per slab of 16, each rounding
+    at most half an ulp of it, uniform up to that: 2^-24 / sqrt(3) rms of the
+    running sum, which grows evenly, so a chain of L / 16 slabs is off by
+    2^-24 / 3 * sqrt(L / 16) of its end (1.3e-6 for all 65536 samples) and s
+    slices' sums by 1 / sqrt(s) of theirs: 1.6e-7 for eight, 2^-24 on top for
+    the slabs' own chains and the adds of the slices."""
+    M, N, K = 1024, 14336, 65536
+    g = torch.Generator(device="cuda").manual_seed(2)
+    A = torch.rand(K, M, device="cuda", generator=g)
+    B = torch.rand(K, N, device="cuda", generator=g)
+    got = _C.matmul(A.t(), B)[:, ::112].double()
+    want = A.double().t() @ B[:, ::112].double()
+    assert float((got - want).norm() / want.norm()) < 1.6e-7 + 2.0 ** -24

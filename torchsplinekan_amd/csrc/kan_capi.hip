@@ -329,7 +329,7 @@ BackwardPlan plan_backward(int64_t n, int64_t I, int64_t O, int64_t G, int64_t k
   p.kaug = I * p.R + (has_base ? I : 0);
   p.need_x = need_x;
   p.need_params = need_params;
-  p.splits = need_params ? gemm_pick_splits<T>(O, p.kaug, n) : 1;
+  p.splits = need_params ? gemm_pick_splits<T>(kLayoutTN, O, p.kaug, n) : 1;
   // transposed weight [kaug, O] (rounded to 256 bytes: E follows it)
   p.waug_elems = need_x ? (size_t)round_up(p.kaug * O, 64) : 0;
   // fp32 with the local basis: dx is contracted inside the input-side GEMM,

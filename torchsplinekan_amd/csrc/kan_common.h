@@ -237,7 +237,7 @@ bool gemm_ecomp_supported(int64_t M, int64_t N, int64_t K, int64_t I, int G, int
 // into C (kan_gemm.hip).  ws must hold matmul_ws_elems(...) elements, with
 // the same max_slice_elems: a non-negative value bounds the split slices'
 // total elements (the allocation-free inference's fixed scratch), -1 leaves
-// the split count to the cost model alone.
+// the split count to the cost model and its longest slices.
 template <typename T>
 int64_t matmul_ws_elems(int layout, int64_t M, int64_t N, int64_t K,
                         int64_t max_slice_elems = -1);
@@ -248,7 +248,7 @@ int launch_matmul(int layout, int64_t M, int64_t N, int64_t K, const T* A, int64
 
 // Split count the GEMM scheduler would choose for a problem (1 = no split).
 template <typename T>
-int gemm_pick_splits(int64_t M, int64_t N, int64_t K, int64_t max_slice_elems = -1);
+int gemm_pick_splits(int layout, int64_t M, int64_t N, int64_t K, int64_t max_slice_elems = -1);
 
 // Estimated seconds of an fp32 product M x N x K as launch_matmul runs it.
 double gemm_seconds_f32(int64_t M, int64_t N, int64_t K);

@@ -1979,10 +1979,28 @@ inline bool gemm_is_thin(int64_t M, int64_t N, int64_t K) {
 // 8 slabs per split; any count, not only powers of two, so that the tiles of
 // all splits fill their last wave of resident blocks.  Long-K products with few output tiles
 // (the parameter product, sample reductions, small-batch inference) split.
+//
+// An fp32 slice is at most kSliceMaxSamples long where both operands are
+// MN-contiguous (sample reductions: long sums with a mean) and kSliceMaxK
+// otherwise, as a sum's error grows with the length of the chain: the
+// parameter product of 65536 samples lay 9.3e-7 off float64 in one chain, 1.2e-7
+// in eight of 8192 (10 intervals; the fp32 MFMA kernel's eight slices 3.1e-7,
+// at 65 intervals its spline columns 1.4e-7 and these 1.2e-7); a forward
+// product over 66600 columns of 4096 -> 256, 13 intervals, 1.2e-6 in one, 0.5e-6
+// in five (fp32 MFMA, nine slices, 0.9e-6).  It costs the partial sums'
+// traffic, about 2 % at most: 1024 x 14336 x 65536 9.0 to 9.3 ms in one slice,
+// 8.9 in eight; x 16384 2.22 and 2.28 ms; 469 x 32130 x 41700 6.40 ms in one,
+// 6.61 in six.
+constexpr int64_t kSliceMaxSamples = 8192;
+constexpr int64_t kSliceMaxK = 16384;
 template <typename T>
-int gemm_pick_splits(int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
+int gemm_pick_splits(int layout, int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
   if (gemm_is_thin(M, N, K)) return K <= kThinMax ? 1 : thin_splits(M, N, K);
   const int64_t cus = device_cu_count();  // (once: the model is evaluated ~200 times)
+  const int64_t least =
+      std::is_same<T, float>::value
+          ? ceil_div(K, layout == kLayoutTN ? kSliceMaxSamples : kSliceMaxK)
+          : 1;
   int best = 1;
   double best_t = 0.0;
   for (int s = 1; s <= 64; ++s) {
@@ -1995,7 +2013,7 @@ int gemm_pick_splits(int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
       if (s > 1 && K / s < 8 * kModelF64[1].bk) break;
       t = est_seconds_f64(kModelF64[pick_cfg_f64(M, N, K, s, cus)], M, N, K, s, cus);
     }
-    if (s == 1 || t < best_t * (1.0 - 1e-9)) {
+    if (s <= least || t < best_t * (1.0 - 1e-9)) {
       best = s;
       best_t = t;
     }
@@ -2007,7 +2025,7 @@ double gemm_seconds_f32(int64_t M, int64_t N, int64_t K) {
   if (gemm_is_thin(M, N, K))  // bound by its largest operand
     return 4.0 * (double)std::max({M * N, M * K, N * K}) / 2e12;
   const int64_t cus = device_cu_count();
-  const int s = gemm_pick_splits<float>(M, N, K, -1);
+  const int s = gemm_pick_splits<float>(kLayoutNT, M, N, K, -1);
   return est_seconds(kModelF32[pick_cfg_f32(M, N, K, s, cus)], M, N, K, s, cus);
 }
 
@@ -2114,9 +2132,8 @@ inline unsigned flat_blocks(int64_t count) {
 
 template <typename T>
 int64_t matmul_ws_elems(int layout, int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
-  (void)layout;
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int s = gemm_pick_splits<T>(M, N, K, max_slice_elems);
+  const int s = gemm_pick_splits<T>(layout, M, N, K, max_slice_elems);
   return s > 1 ? (int64_t)s * M * N : 0;
 }
 
@@ -2130,7 +2147,7 @@ int launch_matmul(int layout, int64_t M, int64_t N, int64_t K, const T* A, int64
                        ldc);
     return check_launch("matmul (K = 0)");
   }
-  const int s = gemm_pick_splits<T>(M, N, K, max_slice_elems);
+  const int s = gemm_pick_splits<T>(layout, M, N, K, max_slice_elems);
   if (s <= 1) return launch_gemm<T>(layout, M, N, K, A, lda, B, ldb, C, ldc, 1, 0, st);
   const int rc = launch_gemm<T>(layout, M, N, K, A, lda, B, ldb, ws, N, s, M * N, st);
   if (rc != KAN_OK) return rc;
@@ -2261,7 +2278,7 @@ template int launch_gemm<float>(int, int64_t, int64_t, int64_t, const float*, in
 template int launch_gemm<double>(int, int64_t, int64_t, int64_t, const double*, int64_t,
                                  const double*, int64_t, double*, int64_t, int, int64_t,
                                  hipStream_t);
-template int gemm_pick_splits<float>(int64_t, int64_t, int64_t, int64_t);
-template int gemm_pick_splits<double>(int64_t, int64_t, int64_t, int64_t);
+template int gemm_pick_splits<float>(int, int64_t, int64_t, int64_t, int64_t);
+template int gemm_pick_splits<double>(int, int64_t, int64_t, int64_t, int64_t);
 
 }  // namespace kan

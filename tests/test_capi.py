@@ -231,3 +231,12 @@ def test_long_fp32_sums_are_split(lib, trans, M, N, K, limit):
     nbytes = ctypes.c_size_t(0)
     lib.check(lib.LIB.kan_hip_matmul_workspace(0, *trans, M, N, K, ctypes.byref(nbytes)))
     assert nbytes.value // (4 * M * N) * limit >= K
+
+
+@pytest.mark.parametrize("trans,M,N,K", [((0, 1), 2000, 131072, 282624),
+                                         ((0, 1), 65536, 65536, 282624),
+                                         ((1, 0), 4096, 57344, 65536)])
+def test_slices_of_long_sums_take_little_memory(lib, trans, M, N, K):
+    nbytes = ctypes.c_size_t(0)
+    lib.check(lib.LIB.kan_hip_matmul_workspace(0, *trans, M, N, K, ctypes.byref(nbytes)))
+    assert nbytes.value <= 1 << 32

@@ -1991,15 +1991,20 @@ inline bool gemm_is_thin(int64_t M, int64_t N, int64_t K) {
 // traffic, about 2 % at most: 1024 x 14336 x 65536 9.0 to 9.3 ms in one slice,
 // 8.9 in eight; x 16384 2.22 and 2.28 ms; 469 x 32130 x 41700 6.40 ms in one,
 // 6.61 in six.
+// What slices are added for this takes at most kSliceElems (4 GiB, 1.5 % of the
+// memory): a large batch of a layer whose weight fills half of it would not fit
+// with 18 slices of its output.
 constexpr int64_t kSliceMaxSamples = 8192;
 constexpr int64_t kSliceMaxK = 16384;
+constexpr int64_t kSliceElems = (int64_t)1 << 30;
 template <typename T>
 int gemm_pick_splits(int layout, int64_t M, int64_t N, int64_t K, int64_t max_slice_elems) {
   if (gemm_is_thin(M, N, K)) return K <= kThinMax ? 1 : thin_splits(M, N, K);
   const int64_t cus = device_cu_count();  // (once: the model is evaluated ~200 times)
   const int64_t least =
       std::is_same<T, float>::value
-          ? ceil_div(K, layout == kLayoutTN ? kSliceMaxSamples : kSliceMaxK)
+          ? std::min(ceil_div(K, layout == kLayoutTN ? kSliceMaxSamples : kSliceMaxK),
+                     kSliceElems / (M * N))
           : 1;
   int best = 1;
   double best_t = 0.0;
@@ -2013,7 +2018,7 @@ int gemm_pick_splits(int layout, int64_t M, int64_t N, int64_t K, int64_t max_sl
       if (s > 1 && K / s < 8 * kModelF64[1].bk) break;
       t = est_seconds_f64(kModelF64[pick_cfg_f64(M, N, K, s, cus)], M, N, K, s, cus);
     }
-    if (s <= least || t < best_t * (1.0 - 1e-9)) {
+    if (s == 1 || s <= least || t < best_t * (1.0 - 1e-9)) {
       best = s;
       best_t = t;
     }

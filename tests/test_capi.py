@@ -240,3 +240,25 @@ def test_slices_of_long_sums_take_little_memory(lib, trans, M, N, K):
     nbytes = ctypes.c_size_t(0)
     lib.check(lib.LIB.kan_hip_matmul_workspace(0, *trans, M, N, K, ctypes.byref(nbytes)))
     assert nbytes.value <= 1 << 32
+
+
+@pytest.mark.parametrize("n,I,O,k", [(1812, 4020, 274269, 2), (12626, 4073, 260184, 3),
+                                     (3349, 2686, 292137, 3), (2060, 3663, 263579, 3),
+                                     (451, 2808, 16123, 3)])
+@pytest.mark.parametrize("base", [0, 1])
+def test_span_products_take_little_more_workspace(lib, n, I, O, k, base):
+    """Where the span-window route would need more workspace than the dense
+    one by over 1 GiB (its transposed weight, a partial dx per output tile)
+    the dense one runs: the call fits where it always did."""
+    def workspace():
+        out = []
+        for fn, flags in ((lib.LIB.kan_hip_infer_workspace, ()),
+                          (lib.LIB.kan_hip_backward_workspace, (1, 0))):
+            nbytes = ctypes.c_size_t(0)
+            lib.check(fn(0, n, I, O, 65, k, base, *flags, ctypes.byref(nbytes)))
+            out.append(nbytes.value)
+        return out
+    auto = workspace()
+    with lib.route("compact_e", 1):      # the dense product
+        dense = workspace()
+    assert all(a <= d + (1 << 30) + 4096 for a, d in zip(auto, dense))

@@ -256,6 +256,9 @@ constexpr double kSpanMargin = 0.8;
 constexpr double kSpanForwardMargin = 0.95;
 constexpr int64_t kSpanForwardMaxO = 256;
 constexpr double kSpanStream = 5e12;  // bytes/s of the passes beside the products
+// Workspace the span products may take whatever the dense ones would: 1 GiB,
+// 0.4 % of the memory.
+constexpr int64_t kSpanWsElems = (int64_t)1 << 28;
 // Forward with the basis kept: the same basis pass and weight packing either way.
 bool span_forward_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
                        SpanPlan* pl) {
@@ -264,19 +267,28 @@ bool span_forward_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, in
   return pl->seconds < kSpanForwardMargin * gemm_seconds_f32(n, O, kaug);
 }
 // Inference: the dense product also writes the basis and reads it back; the
-// span product transposes the packed weight.
+// span product transposes the packed weight.  That copy of the weight may not
+// take more workspace than the basis and the dense product's slices, or than
+// kSpanWsElems: with few samples and a weight of half the memory it would not
+// fit, where the dense product does.
 bool span_infer_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
                      SpanPlan* pl) {
   if (!span_may(n, I, O, R)) return false;
   *pl = span_plan(n, I, O, R, k, false);
+  if (kaug * O + pl->part_elems >
+      std::max(kSpanWsElems, n * kaug + matmul_ws_elems<float>(kLayoutNT, n, O, kaug)))
+    return false;
   return pl->seconds + 8.0 * (double)(kaug * O) / kSpanStream + 4e-6 <
          kSpanMargin * (gemm_seconds_f32(n, O, kaug) + 4.0 * (double)(n * kaug) / kSpanStream);
 }
-// Input gradient: against the dense product and the pass over its windows.
+// Input gradient: against the dense product and the pass over its windows.  A
+// partial dx per output tile may not take more than those windows, or than
+// kSpanWsElems (451 x 2808 -> 16123: 304 MiB for 63).
 bool span_dx_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t kaug,
                   SpanPlan* pl) {
   if (!span_may(n, I, O, R)) return false;
   *pl = span_plan(n, I, O, R, k, true);
+  if (pl->part_elems > std::max(kSpanWsElems, n * I * (k + 1))) return false;
   return pl->seconds < kSpanMargin * (gemm_seconds_f32(n, kaug, O) +
                                       4.0 * (double)(n * I * (k + 4)) / 3e12);
 }

@@ -521,8 +521,10 @@ SpanPlan span_plan(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, bool d
   p.tiles_o = ceil_div(O, (int64_t)(64 * p.v));
   const int64_t chunks = ceil_div(I, (int64_t)kSpanChunk);
   double best = 0.0;
-  // (forward slices leave partial sums: at most 24 of them)
+  // (forward slices leave partial sums: at most 24 of them, and no more than
+  // the basis would take)
   for (int64_t s = 1; s <= (dx ? 64 : 24) && s <= chunks; ++s) {
+    if (!dx && s > 1 && s * O > I * (R + 1)) break;
     const int64_t per = ceil_div(chunks, s);
     if (s > 1 && (per < 4 || ceil_div(chunks, per) != s)) continue;
     const double rounds = (double)ceil_div(p.tiles_n * p.tiles_o * s, cus);
@@ -544,7 +546,6 @@ SpanPlan span_plan(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, bool d
   const int64_t parts = dx ? p.tiles_o : p.slices;
   p.part_elems = parts > 1 ? parts * n * (dx ? I : O) : 0;
   if (dx && parts > 1) p.seconds += 8.0 * (double)p.part_elems / 5e12;
-  (void)R;
   (void)k;
   return p;
 }

@@ -19,14 +19,49 @@ def _operands(M, N, K, ta, tb, seed=0):
     return (A.t() if ta else A), (B.t() if tb else B)
 
 
-def _check(A, B):
+def _check(A, B, adds=None):
     got = _C.matmul(A.cuda(), B.cuda()).cpu().double()
     want = A.double() @ B.double()
-    # one rounding per slab, at most 16 in a slab's chain (six MFMAs, each two
-    # truncating steps, and the dropped products), of 2^-24 of the sum of
-    # magnitudes; 64 more for the split slices
-    bound = (A.shape[1] / 16 + 16 + 64) * 2.0 ** -24 * (A.double().abs() @ B.double().abs())
+    adds = A.shape[1] / 16 if adds is None else adds
+    # one rounding per add (a slab's, K / 16 of them), at most 16 in a slab's
+    # chain (six MFMAs, each two truncating steps, and the dropped products), of
+    # 2^-24 of the sum of magnitudes
+    bound = (adds + 16) * 2.0 ** -24 * (A.double().abs() @ B.double().abs())
     assert bool(((got - want).abs() <= bound).all())
+    # Normwise: adds to a sum that grows with their square root, each off by at
+    # most 2^-24 / sqrt(3) rms of it, make sqrt(adds / 2) of that (1.4e-7 at
+    # K = 530); a slab's last MFMA truncates its own sum (2^-23 / sqrt(3) of it,
+    # whatever K) and the earlier ones at most half as much more.  An operand
+    # without its lo part costs 2e-6, a missing mid times mid product 6e-7.
+    rel = 2.0 ** -24 / 3 ** 0.5 * ((adds / 2) ** 0.5 + 2 * 1.5)
+    assert float((got - want).norm() / want.norm()) <= rel
+
+
+@pytest.mark.parametrize("tile", ["256", "128", "256x64"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False), (False, False), (True, True)])
+def test_every_part_product_decides(tile, ta, tb):
+    """Sums in which all but one of the six part products cancel: 2^-20 from
+    lo times hi, hi times lo or mid times mid, 2^-10 from mid times hi or hi
+    times mid, 1 from hi times hi.  A row holds one such sum, in one 8-k half of
+    one of 18 slabs (either side of the change of sign), and is zero elsewhere;
+    every value is exact."""
+    e10, e20 = 2.0 ** -10, 2.0 ** -20
+    sums = [([1 + e10 + e20, -(1 + e10)], [1, 1]), ([1, -1], [1 + e10 + e20, 1 + e10]),
+            ([1 + e10, -1, -1], [1 + e10, 1, 2 * e10]), ([1 + e10, -1], [1, 1]),
+            ([1, -1], [1 + e10, 1]), ([1], [1])]
+    slabs, N = 18, 64
+    for a, b in sums:
+        A, B = torch.zeros(2 * slabs, 16 * slabs), torch.zeros(16 * slabs, N)
+        want = sum(u * v for u, v in zip(a, b))
+        for r in range(2 * slabs):
+            for i, (u, v) in enumerate(zip(a, b)):
+                k = 8 * r + (3 * r + i) % 8
+                A[r, k], B[k] = u, v
+        A = A.t().contiguous().t() if ta else A
+        B = B.t().contiguous().t() if tb else B
+        with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
+            got = _C.matmul(A.cuda(), B.cuda()).cpu()
+        assert bool((got == want).all())
 
 
 @pytest.mark.parametrize("tile", ["256", "128", "256x64"])
@@ -103,7 +138,8 @@ def test_small_and_large_products(tile, ta, tb, pa, pb):
     parts overflow are evaluated in plain fp32)."""
     A, B = _operands(70, 40, 100, ta, tb, seed=pa)
     with _lib.route("gemm_tile", _lib.GEMM_TILES[tile]):
-        _check(A.clamp(-1.9, 1.9) * 2.0 ** pa, B * 2.0 ** pb)
+        # (plain fp32 adds one product at a time)
+        _check(A.clamp(-1.9, 1.9) * 2.0 ** pa, B * 2.0 ** pb, None if pa < 0 else 100)
 
 
 @pytest.mark.parametrize("tile", ["256", "128", "256x64"])
@@ -133,15 +169,25 @@ def test_error_has_no_mean():
     assert abs(float(err.mean())) < limit
 
 
-def test_leading_dimension_past_a_buffer_resource():
-    """256 rows of 2.2 million columns span more than 2^31 bytes: the loads
-    with 64-bit addresses."""
-    M, N, K = 300, 70, 150
-    wide = torch.empty(M, 2_200_000, device="cuda")
-    A, B = _operands(M, N, K, False, True, seed=5)
-    wide[:, :K] = A.cuda()
-    got = _C.matmul(wide[:, :K], B.cuda())
-    assert torch.equal(got, _C.matmul(A.cuda(), B.cuda()))
+@pytest.mark.parametrize("kcont_a,kcont_b", [(True, False), (True, True), (False, False),
+                                             (False, True)])
+def test_leading_dimension_past_a_buffer_resource(kcont_a, kcont_b):
+    """256 rows of 2.2 million columns, or 16 of 34 million, span more than 2^31
+    bytes: the loads with 64-bit addresses."""
+    M, N, K = 300, 70, 40
+    A, B = _operands(M, N, K, not kcont_a, kcont_b, seed=5)
+    if kcont_a:
+        wide = torch.empty(M, 2_200_000, device="cuda")[:, :K]
+    else:
+        wide = torch.empty(K, 34_000_000, device="cuda")[:, :M].t()
+    wide.copy_(A)
+    with _lib.route("gemm_tile", 0):    # 256 rows
+        got = _C.matmul(wide, B.cuda())
+        assert torch.equal(got, _C.matmul(A.cuda(), B.cuda()))
+        _check(wide.cpu(), B)
+        # the wide operand on the other side
+        assert torch.equal(_C.matmul(B.cuda().t(), wide.t()),
+                           _C.matmul(B.cuda().t(), A.cuda().t()))
 
 
 def test_long_sums_of_samples():

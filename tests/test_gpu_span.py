@@ -15,12 +15,24 @@ from torchsplinekan_amd.reference_backend import compute_basis
 
 pytestmark = pytest.mark.gpu
 
-# n, I, O, G, k, base: shapes whose inference or input gradient (or both) the
-# rule gives to the span kernels
-SHAPES = [(8498, 187, 51, 65, 2, True), (3000, 333, 61, 66, 2, True),
-          (3001, 250, 259, 65, 3, False), (13220, 73, 19, 65, 1, True),
-          (1281, 1068, 461, 65, 1, True), (4500, 500, 61, 65, 2, False),
-          (4729, 948, 61, 65, 3, True)]
+# (n, I, O, G, k, base) and which of the forward, the inference and the input
+# gradient the rule gives to the span kernels there: each of 1, 2 and 4 outputs
+# a lane (O up to 64, up to 128, more), with rows staged 16 bytes at a time (O a
+# multiple of 4) and value by value, at every order
+SHAPES = [((8498, 187, 51, 65, 2, True), (1, 1, 0)), ((3000, 333, 61, 66, 2, True), (0, 1, 0)),
+          ((3001, 250, 259, 65, 3, False), (0, 1, 0)), ((13220, 73, 19, 65, 1, True), (0, 1, 0)),
+          ((1281, 1068, 461, 65, 1, True), (0, 0, 1)), ((4500, 500, 61, 65, 2, False), (1, 1, 1)),
+          ((4729, 948, 61, 65, 3, True), (1, 1, 1)), ((5115, 253, 64, 65, 1, True), (1, 1, 1)),
+          ((1798, 853, 64, 65, 2, True), (1, 1, 1)), ((2681, 478, 64, 65, 3, False), (1, 1, 1)),
+          ((5565, 251, 96, 65, 1, True), (1, 1, 0)), ((2315, 594, 96, 65, 3, True), (1, 1, 0)),
+          ((2191, 544, 100, 65, 1, True), (0, 1, 1)), ((4784, 297, 100, 65, 2, False), (1, 1, 0)),
+          ((1193, 993, 100, 65, 3, True), (0, 0, 1)), ((1723, 714, 101, 65, 1, False), (0, 1, 1)),
+          ((3154, 460, 101, 65, 2, False), (1, 1, 0)), ((2103, 971, 101, 65, 3, False), (0, 1, 1)),
+          ((1949, 696, 101, 65, 3, True), (1, 1, 0)), ((2777, 652, 127, 65, 3, True), (1, 1, 1)),
+          ((3144, 472, 128, 65, 1, True), (1, 1, 1)), ((2001, 911, 128, 65, 2, False), (1, 1, 1)),
+          ((2416, 593, 128, 65, 3, True), (1, 1, 1)), ((3862, 336, 256, 65, 1, True), (1, 1, 1)),
+          ((2168, 582, 256, 65, 2, False), (1, 1, 1)), ((6061, 212, 256, 65, 3, True), (1, 1, 1)),
+          ((1418, 668, 384, 65, 2, True), (0, 0, 1))]
 
 
 def _workspace(fn, *args):
@@ -30,15 +42,16 @@ def _workspace(fn, *args):
 
 
 def _routes(n, I, O, G, k, base):
-    """Which of (inference, input gradient) run on the span kernels: those
-    whose workspace differs from the dense route's."""
+    """Which of (forward, inference, input gradient) run on the span kernels:
+    those whose workspace differs from the dense route's."""
     out = []
-    for fn, args in ((_lib.LIB.kan_hip_infer_workspace, (0, n, I, O, G, k, int(base))),
+    for fn, args in ((_lib.LIB.kan_hip_forward_workspace, (0, n, I, O, G, k, int(base))),
+                     (_lib.LIB.kan_hip_infer_workspace, (0, n, I, O, G, k, int(base))),
                      (_lib.LIB.kan_hip_backward_workspace, (0, n, I, O, G, k, int(base), 1, 0))):
         auto = _workspace(fn, *args)
         with _lib.route("compact_e", 1):
-            out.append(auto != _workspace(fn, *args))
-    return out
+            out.append(int(auto != _workspace(fn, *args)))
+    return tuple(out)
 
 
 def _layer(n, I, O, G, k, base, seed=0):
@@ -57,10 +70,10 @@ def _norm(u, v):
     return float((u - v).norm() / v.norm())
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_span_products_match_float64(shape):
+@pytest.mark.parametrize("shape,routes", SHAPES)
+def test_span_products_match_float64(shape, routes):
     n, I, O, G, k, base = shape
-    assert any(_routes(*shape))
+    assert _routes(*shape) == routes
     x, grid, bw, sw, sc = _layer(*shape)
     D = torch.randn(n, O, generator=torch.Generator().manual_seed(1)).cuda()
     xg = x.clone().requires_grad_()
@@ -96,7 +109,7 @@ def test_span_inputs_and_weights_that_are_not_finite():
     silu alone; a weight that is not finite reaches its output's every sample,
     times the sample's basis value or silu, or times zero."""
     shape = (3000, 333, 61, 66, 2, True)
-    assert _routes(*shape)[0]
+    assert _routes(*shape)[1]
     x, grid, bw, sw, sc = _layer(*shape)
     bw = bw.abs() + 0.1
     x[5, 7], x[6, 8], x[7, 9], x[8, 10], x[9, 50] = float("nan"), float("inf"), 50.0, 0.0, -50.0
@@ -120,7 +133,7 @@ def test_span_input_gradient_of_values_that_are_not_finite(shape):
     """As from the dense product's window rows: an x outside the knots meets
     no spline weight and, without a base branch, no dL/dy."""
     n, I, O, G, k, base = shape
-    assert _routes(*shape)[1]
+    assert _routes(*shape)[2]
     x, grid, bw, sw, sc = _layer(*shape)
     D = torch.randn(n, O, generator=torch.Generator().manual_seed(1)).cuda()
     x[0:3] = 40.0                        # outside every feature's knots
@@ -148,7 +161,7 @@ def test_span_input_gradient_of_values_that_are_not_finite(shape):
 
 def test_span_products_in_a_captured_graph():
     n, I, O, G, k, base = shape = (4729, 948, 61, 65, 3, True)
-    assert all(_routes(*shape))
+    assert _routes(*shape) == (1, 1, 1)
     x, grid, bw, sw, sc = _layer(*shape)
     D = torch.randn(n, O, device="cuda")
     xg = x.clone().requires_grad_()

@@ -251,10 +251,18 @@ bool span_may(int64_t n, int64_t I, int64_t O, int64_t R) {
 //    against 6.85 and 4.24 against 7.64 ms), lost up to 10 % at 0.95;
 //  * the forward that keeps the basis up to 256 outputs, below 0.95: won by 1.04
 //    to 1.4 times (8192 x 4096 -> 256: 3.65 against 5.10 ms); above 256 outputs
-//    it lost up to 14 % (332 x 1699 -> 1038: 0.87 against 0.75 ms).
+//    it lost up to 14 % (332 x 1699 -> 1038: 0.87 against 0.75 ms);
+//  * that forward of at most 16 outputs below 0.73, as its dense product runs on
+//    the thin kernels: won by 1.09 to 1.66 times there, between 0.75 and 0.95 lost
+//    up to 21 % (921 x 1972 -> 13: 0.41 against 0.33 ms).  The dense input
+//    gradient of so few outputs runs on the tiles all the same, and is estimated
+//    as that: by the thin kernels' rate the span kernel was taken where it lost
+//    up to 42 % (6879 x 470 -> 9: 0.34 against 0.20 ms).
 constexpr double kSpanMargin = 0.8;
 constexpr double kSpanForwardMargin = 0.95;
 constexpr int64_t kSpanForwardMaxO = 256;
+constexpr int64_t kSpanThinO = 16;
+constexpr double kSpanThinForwardMargin = 0.73;
 constexpr double kSpanStream = 5e12;  // bytes/s of the passes beside the products
 // Workspace the span products may take whatever the dense ones would: 1 GiB,
 // 0.4 % of the memory.
@@ -264,7 +272,8 @@ bool span_forward_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, in
                        SpanPlan* pl) {
   if (O > kSpanForwardMaxO || !span_may(n, I, O, R)) return false;
   *pl = span_plan(n, I, O, R, k, false);
-  return pl->seconds < kSpanForwardMargin * gemm_seconds_f32(n, O, kaug);
+  return pl->seconds < (O <= kSpanThinO ? kSpanThinForwardMargin : kSpanForwardMargin) *
+                           gemm_seconds_f32(n, O, kaug);
 }
 // Inference: the dense product also writes the basis and reads it back; the
 // span product transposes the packed weight.  That copy of the weight may not
@@ -289,7 +298,7 @@ bool span_dx_wins(int64_t n, int64_t I, int64_t O, int64_t R, int64_t k, int64_t
   if (!span_may(n, I, O, R)) return false;
   *pl = span_plan(n, I, O, R, k, true);
   if (pl->part_elems > std::max(kSpanWsElems, n * I * (k + 1))) return false;
-  return pl->seconds < kSpanMargin * (gemm_seconds_f32(n, kaug, O) +
+  return pl->seconds < kSpanMargin * (gemm_ecomp_seconds(n, kaug, O) +
                                       4.0 * (double)(n * I * (k + 4)) / 3e12);
 }
 

@@ -252,6 +252,9 @@ int gemm_pick_splits(int layout, int64_t M, int64_t N, int64_t K, int64_t max_sl
 
 // Estimated seconds of an fp32 product M x N x K as launch_matmul runs it.
 double gemm_seconds_f32(int64_t M, int64_t N, int64_t K);
+// The same of the compact input-side product (launch_gemm_ecomp), which runs on
+// the tiles, unsplit, at any K.
+double gemm_ecomp_seconds(int64_t M, int64_t N, int64_t K);
 
 // Span-window products of a layer with many basis functions per feature
 // (kan_span.hip): y and dx from x, the knots and the transposed augmented

@@ -1,6 +1,6 @@
-"""GPU parity at BASELINE.json's workloads themselves, built by the same
+"""GPU parity at the benchmark's workloads themselves, built by the same
 functions bench.py times (bench.build_c2 .. build_c5), against the fp64
-oracle at the north star's fp32 bar (normwise relative 1e-5):
+oracle at the fp32 parity bar (normwise relative 1e-5):
 
 * c3: KANLinear 1024 -> 1024 G10 k3, N = 65536, x with grad: every element
   of y, dx, dcoef, dscaler and dbase_w (tests/_fullcheck.py: the oracle in

@@ -20,7 +20,8 @@
 // the two by half: 64 and 74 clocks measured.  At 8192 x 4096 -> 256, R = 68:
 // forward 3.65 ms against 5.10 ms for the split-bf16 product over all columns
 // (which also needs the basis written, 1.73 ms), input gradient 4.23 against
-// 7.31 + 0.33 ms (compact product and its window pass).
+// 7.31 + 0.33 ms (compact product and its window pass), timed alone (3.9 and
+// 4.4 ms within a training step).
 //
 // Layout: 8 waves of 24 (input: 20) samples share the weight rows of one feature and
 // 64 V outputs (V per lane), double buffered in LDS while the next feature's
@@ -585,7 +586,7 @@ int launch_span_forward(const SpanPlan& pl, const float* x, const float* grid, c
   p.out_stride = n * O;
   {
     TimedLaunch timed(kClassContraction, st,
-                      2.0 * (double)n * (double)O * (double)I * (p.R + (base ? 1 : 0)));
+                      2.0 * (double)n * (double)O * (double)I * (k + 1 + (base ? 1 : 0)));
     const int rc = launch_span<false>(p, k, pl.v, st);
     if (rc != KAN_OK) return rc;
   }
@@ -601,7 +602,7 @@ int launch_span_dx(const SpanPlan& pl, const float* D, const float* x, const flo
   p.out_stride = n * I;
   {
     TimedLaunch timed(kClassContraction, st,
-                      2.0 * (double)n * (double)O * (double)I * (p.R + (base ? 1 : 0)));
+                      2.0 * (double)n * (double)O * (double)I * (k + 1 + (base ? 1 : 0)));
     const int rc = launch_span<true>(p, k, pl.v, st);
     if (rc != KAN_OK) return rc;
   }

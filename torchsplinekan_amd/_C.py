@@ -37,7 +37,8 @@ def _req(cond: bool, *msg) -> None:
 def _check_inputs(x, grid, base_weight, spline_weight, spline_scaler, spline_order, has_scaler):
     """Validation of kan_check_inputs (csrc/kan_ops.h:27-78) with the same
     messages.  The reference's 32-bit index guard (B*I*(G+2k) <= INT_MAX) is
-    not applied: every native kernel here uses 64-bit offsets."""
+    not applied: the native kernels use 64-bit offsets, and 32-bit ones only
+    within a tile that the host has found to span less than 2^31 bytes."""
     _req(x.dim() == 2, "x must be 2-D [B, I], got ", x.dim(), "-D")
     _req(grid.dim() == 2, "grid must be 2-D [I, G+2k+1]")
     _req(spline_weight.dim() == 3, "spline_weight must be 3-D [O, I, R]")

@@ -242,8 +242,9 @@ bool span_may(int64_t n, int64_t I, int64_t O, int64_t R) {
          kan_hip_get_route(KAN_ROUTE_FUSED_DX) == 0 &&
          kan_hip_get_route(KAN_ROUTE_GEMM_TILE) == -1;
 }
-// Where the lines lie (64 random layers of 23 to 68 basis functions, both ways
-// measured; the two estimates together are off by up to 20 %):
+// Where the lines lie (random layers of 23 to 68 basis functions, both ways
+// measured, 64 of them in profiles/span_rule_sweep.txt; the two estimates
+// together are off by up to 20 %):
 //  * rows below 40 stay dense (at 23 the input gradient lost up to 28 %: 16628 x
 //    3297 -> 22, 2.71 against 1.95 ms);
 //  * inference and input gradient below 0.8 of the dense estimate: won by 1.03

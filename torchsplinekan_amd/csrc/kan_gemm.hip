@@ -768,16 +768,20 @@ struct EpiSide {
 //
 // An fp32 value times 2^24 is the sum of three bf16 values, hi + mid + lo,
 // exactly (8 significant bits each, every part rounded to nearest, so mid <=
-// 2^-9 and lo <= 2^-18 of it).  The factor takes fp32's last bit, 2^-149, to
-// 2^-125, so that no part is a subnormal bf16 value: without it an operand
-// below 2^-110 lost its low parts (1e-37 times 1e30 came out 5e-4 off).  It stands where A's sign is set anyhow, so B
-// alone pays for it, one VALU operation a value (forward 65536 x 1024 x 14336
-// 8.78 -> 8.90 ms, input-side and parameter products within 1 %, 5003 x 77 x
-// 3311 54 -> 57 us); the sums are scaled back as they are stored.  A product of two such sums needs six bf16 products
-// to fp32 accuracy (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three
-// dropped ones are below 2^-26 of the product.  Every product of two bf16
+// 2^-9 and lo <= 2^-18 of it).  A product of two such sums needs six bf16
+// products to fp32 accuracy (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the
+// three dropped ones are below 2^-26 of the product.  (The method is that of
+// Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence
+// Datatype For Higher-Precision Computations", 2019.)  A product of two bf16
 // values is exact in fp32 and the MFMA accumulates in fp32, so the result
 // carries the accumulation's rounding only.
+//
+// Scale: the factor takes fp32's last bit, 2^-149, to 2^-125, so that no part
+// is a subnormal bf16 value; without it an operand below 2^-110 lost its low
+// parts (1e-37 times 1e30 came out 5e-4 off).  It stands where A's sign is set
+// anyhow, so B alone pays for it, one VALU operation a value (5003 x 77 x 3311
+// 39 -> 42 us, the large products below within 1 %); the sums are scaled back
+// as they are stored.
 //
 // Accumulation: a 16-k slab's six MFMAs of a tile run as one chain from zero
 // (smallest parts first) and their result is added to the tile's sum, so the
@@ -786,6 +790,7 @@ struct EpiSide {
 // values non-zero (a basis operand) was more than the fp32 MFMA's one per
 // non-zero k: relative error against float64 1.73e-6, fp32 MFMA 1.32e-6, as
 // built 0.58e-6 (K = 1024, dense: 0.48, 0.58 and 0.16e-6).  The adds cost 5 %.
+// How long a sum may grow is gemm_pick_splits' to say.
 //
 // Sign: the bf16 MFMA rounds its aligned terms towards minus infinity, so its
 // error has a mean, -3e-8 of a term per slab, that grows with the number of
@@ -798,23 +803,26 @@ struct EpiSide {
 // (Subtracting every second slab's partial sum, an FMA by +-1, cost 5 %;
 // turning the sums costs one VALU operation a value every 16 slabs, 1.5 %.)
 //
-// What bounds it: the chip's power.  At 65536 x 1024 x 14336 the kernel runs
-// at 1.9 GHz (the fp32 MFMA kernel before it at 2.37) with the MFMA pipes 0.70
-// busy: 1.35 PFLOP/s of bf16, about what torch.mm reaches in bf16 on the same
-// card (1.17-1.41).  Measured against the fp32 MFMA kernel on one box:
-// forward 65536 x 1024 x 14336 12.63 -> 8.59 ms, input-side 65536 x 14336 x
-// 1024 13.09 -> 9.47, parameter 1024 x 14336 x 65536 12.71 -> 8.77 (152 ->
-// 224, 147 -> 203, 151 -> 219 TFLOP/s of fp32 work); odd sizes, 1000^3 with
-// K % 16 != 0: 0.143 -> 0.055 ms.
+// What bounds it: MFMA issue and the clock.  At 65536 x 1024 x 14336 the chip
+// holds 1.7 to 1.9 GHz (2.37 under the fp32 MFMA kernel before it), which caps
+// the bf16 MFMAs at 1.9 PFLOP/s, and the MFMA pipes are busy for 0.63 to 0.68
+// of those cycles (the VALU, which splits, for 0.51 to 0.53): 1.33 PFLOP/s of
+// bf16, where torch.mm reaches 1.17 to 1.41 on the same card.  Measured against
+// the fp32 MFMA kernel on one box: forward 65536 x 1024 x 14336 12.69 -> 8.64
+// ms, input-side 65536 x 14336 x 1024 13.15 -> 9.46, parameter 1024 x 14336 x
+// 65536 12.89 -> 8.88 (152 -> 223, 146 -> 203, 149 -> 217 TFLOP/s of fp32
+// work); odd sizes, 1000 x 1000 x 1003: 0.059 -> 0.034 ms.
 //
 // Layout: operands are split on their way from registers to LDS (5.5 VALU
-// operations a value and one to scale it, hidden behind the MFMAs), so global
-// memory holds fp32 only and either global layout becomes the K-contiguous
-// rows the MFMA reads with 16-byte loads.  Slabs are one MFMA deep (16 k; 48 KB for 256 + 256
-// rows) and double buffered.  Per slab a wave keeps B's fragments and two
+// operations a value and one to scale it, beside the MFMAs), so global memory
+// holds fp32 only and either global layout becomes the K-contiguous rows the
+// MFMA reads with 16-byte loads.  Slabs are one MFMA deep (16 k; 48 KB for 256
+// + 256 rows) and double buffered.  Per slab a wave keeps B's fragments and two
 // rows of A's; a slab's stores, the loads of the slab after next and the
 // adds are spread over its tiles, and the barrier that publishes the next
 // slab sits before the last tile, whose MFMAs cover the next first reads.
+// (What the compiler spills of the 256 x 256 tile belongs to the loop with
+// 64-bit addresses; the buffer-load loop reloads two values a slab.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -1376,7 +1384,8 @@ bool vec_ok(const T* ptr, int64_t ld) {
 // three products of 784 -> 256, 256 -> 256, 1024 -> 1024, 512 -> 512, 512 ->
 // 64 and 4096 -> 256 layers, small batches and odd sizes (fit error 8 % rms
 // for the first two, 12 % for the narrow one; the choice it makes costs at
-// most 11 % over the best of the sweep, 2 % on average).  The dispatcher
+// most 6 % over the best of the sweep, 1 % on average:
+// profiles/gemm_split_sweep.txt).  The dispatcher
 // spreads workgroups over CUs, so the busiest CU runs ceil(tiles / CUs)
 // blocks one after another (two small blocks that share a CU run at half
 // speed each, the same total); a block costs its MFMA work at the

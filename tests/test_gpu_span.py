@@ -12,6 +12,7 @@ import torch.nn.functional as F
 
 from torchsplinekan_amd import _C, _lib
 from torchsplinekan_amd.reference_backend import compute_basis
+from tests._util import make_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -93,6 +94,35 @@ def test_span_products_match_float64(shape, routes):
     assert _norm(yi, want.detach()) < 1e-5
     assert _norm(dx, wdx) < 1e-5
     assert torch.equal(yi, _C.kan_infer(x, grid, waug, k, base))    # fixed order of sums
+
+
+@pytest.mark.parametrize("shape", [(5115, 253, 64, 65, 1, True), (2001, 911, 128, 65, 2, True),
+                                   (4729, 948, 61, 65, 3, True)])
+def test_span_products_of_repeated_knots(shape):
+    """Knots of up to full multiplicity, inside and at both ends, and an x on
+    every knot, against the dense route."""
+    n, I, O, G, k, base = shape
+    assert _routes(*shape) == (1, 1, 1)
+    x, _, bw, sw, sc = _layer(*shape)
+    grid = make_grid(I, G, k, "repeated", seed=1)
+    grid[:, 10:11 + k] = grid[:, 10:11]
+    grid[:, :k + 1], grid[:, -k - 1:] = grid[:, k:k + 1], grid[:, -k - 1:-k]
+    grid = grid.float().cuda()
+    x = (x + 1) / 2 * (grid.max() - grid.min()) + grid.min()
+    x[:grid.shape[1]] = grid.t()
+    D = torch.randn(n, O, generator=torch.Generator().manual_seed(1)).cuda()
+    waug = _C.pack_weight(bw, sw, sc, k, True)
+
+    def products():
+        xg = x.clone().requires_grad_()
+        y = _C.kan_apply(xg, grid, bw, sw, sc, k, True)
+        return y, _C.kan_infer(x, grid, waug, k, base), torch.autograd.grad(y, xg, D)[0]
+
+    got = products()
+    with _lib.route("compact_e", 1):
+        want = products()
+    for u, v in zip(got, want):
+        assert bool(u.isfinite().all()) and _norm(u, v.detach().double()) < 1e-5
 
 
 def _same_classes(y, want):
